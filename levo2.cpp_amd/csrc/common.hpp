@@ -57,7 +57,7 @@ int dequantize_kquant(levo_hip_type type, const void * src, void * dst, levo_hip
 constexpr int kNotFused = 1;
 
 // Device memory a launch may overwrite (null: none).
-struct scratch {
+struct scratch_span {
     float * p;
     int64_t floats;
 };
@@ -70,16 +70,16 @@ struct scratch {
 int decoder_conv1d(const float * x, int64_t c_in, int64_t t, const void * alpha_log, const void * beta_log,
                    levo_hip_type param_type, const float * weight, int64_t c_out, int64_t kernel, const float * bias,
                    int64_t padding, int64_t dilation, const float * residual, float * y, const void * post_alpha_log,
-                   const void * post_beta_log, scratch ws, scratch pack, hipStream_t stream);
+                   const void * post_beta_log, scratch_span ws, scratch_span pack, hipStream_t stream);
 // levo_hip_snake_conv_transpose1d_split on contiguous rows, likewise.
 int decoder_upsample(const float * x, int64_t c_in, int64_t t, const void * alpha_log, const void * beta_log,
                      levo_hip_type param_type, const float * packed_weight, int64_t c_out, int64_t stride,
-                     const float * bias, int64_t padding, float * y, scratch ws, scratch pack, hipStream_t stream);
+                     const float * bias, int64_t padding, float * y, scratch_span ws, scratch_span pack, hipStream_t stream);
 int launch_residual_unit_fused(const float * x, int64_t c, int64_t t, const void * pre_alpha_log,
                                const void * pre_beta_log, const float * w0, const float * b0,
                                const void * post_alpha_log, const void * post_beta_log, const float * w1,
                                const float * b1, int64_t dilation, levo_hip_type param_type, float * y,
-                               const scratch & pack, hipStream_t stream);
+                               const scratch_span & pack, hipStream_t stream);
 
 inline bool aligned16(const void * p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 

@@ -1321,7 +1321,7 @@ int launch_residual_unit_fused(const float * x, int64_t c, int64_t t, const void
                                const void * pre_beta_log, const float * w0, const float * b0,
                                const void * post_alpha_log, const void * post_beta_log, const float * w1,
                                const float * b1, int64_t dilation, levo_hip_type param_type, float * y,
-                               const scratch & pack, hipStream_t st) {
+                               const scratch_span & pack, hipStream_t st) {
     if (c != kMT || dilation < 1 || !aligned16(w0) || !aligned16(w1) || pre_alpha_log == nullptr ||
         pre_beta_log == nullptr || post_alpha_log == nullptr || post_beta_log == nullptr)
         return kNotFused;
@@ -1467,7 +1467,7 @@ double f32_launch_us(int kw, int64_t wgs, int64_t splits, int64_t c_in) {
 }
 
 int try_x3(const conv_params & p, int kw, int64_t wgs, int64_t splits, float * ws, int64_t ws_floats,
-           const scratch & pack, hipStream_t st, const char * what) {
+           const scratch_span & pack, hipStream_t st, const char * what) {
     const x3_conv c = x3_of(p);
     const int64_t bytes = x3_pack_bytes(c, kw);
     if (bytes < 0) return kNotX3;
@@ -1496,7 +1496,7 @@ int conv1d_entry(const float * x, int64_t x_stride, int64_t c_in, int64_t t_in, 
                  const void * beta_log, levo_hip_type param_type, const float * weight, int64_t c_out,
                  int64_t kernel, const float * bias, int64_t padding, int64_t dilation, const float * residual,
                  int64_t residual_stride, float * y, int64_t y_stride, float * ws, int64_t ws_floats,
-                 const scratch & pack, const void * post_alpha_log, const void * post_beta_log, hipStream_t st,
+                 const scratch_span & pack, const void * post_alpha_log, const void * post_beta_log, hipStream_t st,
                  const char * what) {
     LEVO_REQUIRE(c_in > 0 && c_out > 0 && t_in > 0, "LeVo audio graph: incompatible Conv1d weight/input shapes");
     LEVO_REQUIRE(padding >= 0 && dilation > 0, "LeVo audio graph: invalid Conv1d stride, padding, or dilation");
@@ -1602,7 +1602,7 @@ extern "C" int levo_hip_snake_conv1d(const float * x, int64_t x_stride, int64_t 
                                      int64_t residual_stride, float * y, int64_t y_stride,
                                      levo_hip_stream_t stream) {
     return conv1d_entry(x, x_stride, c_in, t_in, alpha_log, beta_log, param_type, weight, c_out, kernel, bias,
-                        padding, dilation, residual, residual_stride, y, y_stride, nullptr, 0, scratch{}, nullptr, nullptr,
+                        padding, dilation, residual, residual_stride, y, y_stride, nullptr, 0, scratch_span{}, nullptr, nullptr,
                         as_hip(stream), "levo_hip_snake_conv1d");
 }
 
@@ -1611,7 +1611,7 @@ namespace levo_hip {
 int decoder_conv1d(const float * x, int64_t c_in, int64_t t, const void * alpha_log, const void * beta_log,
                    levo_hip_type param_type, const float * weight, int64_t c_out, int64_t kernel, const float * bias,
                    int64_t padding, int64_t dilation, const float * residual, float * y, const void * post_alpha_log,
-                   const void * post_beta_log, scratch ws, scratch pack, hipStream_t st) {
+                   const void * post_beta_log, scratch_span ws, scratch_span pack, hipStream_t st) {
     return conv1d_entry(x, t, c_in, t, alpha_log, beta_log, param_type, weight, c_out, kernel, bias, padding,
                         dilation, residual, residual ? t : 0, y, t, ws.p, ws.floats, pack, post_alpha_log,
                         post_beta_log, st, "levo_hip_vae_decode");
@@ -1633,7 +1633,7 @@ extern "C" int levo_hip_snake_conv1d_split(const float * x, int64_t x_stride, in
                                            levo_hip_stream_t stream) {
     return conv1d_entry(x, x_stride, c_in, t_in, alpha_log, beta_log, param_type, weight, c_out, kernel, bias,
                         padding, dilation, residual, residual_stride, y, y_stride, workspace, workspace_floats,
-                        scratch{}, nullptr, nullptr, as_hip(stream), "levo_hip_snake_conv1d_split");
+                        scratch_span{}, nullptr, nullptr, as_hip(stream), "levo_hip_snake_conv1d_split");
 }
 
 namespace levo_hip {
@@ -1676,7 +1676,7 @@ namespace {
 int conv_transpose_entry(const float * x, int64_t x_stride, int64_t c_in, int64_t t_in, const void * alpha_log,
                          const void * beta_log, levo_hip_type param_type, const float * packed_weight,
                          int64_t c_out, int64_t stride, const float * bias, int64_t padding, float * y,
-                         int64_t y_stride, float * ws, int64_t ws_floats, const scratch & pack, hipStream_t st,
+                         int64_t y_stride, float * ws, int64_t ws_floats, const scratch_span & pack, hipStream_t st,
                          const char * what) {
     LEVO_REQUIRE(c_in > 0 && c_out > 0 && t_in > 0, "LeVo audio graph: incompatible ConvTranspose1d weight/input shapes");
     LEVO_REQUIRE(stride > 0 && padding >= 0, "LeVo audio graph: invalid ConvTranspose1d stride or padding");
@@ -1755,7 +1755,7 @@ int conv_transpose_entry(const float * x, int64_t x_stride, int64_t c_in, int64_
 
 int decoder_upsample(const float * x, int64_t c_in, int64_t t, const void * alpha_log, const void * beta_log,
                      levo_hip_type param_type, const float * packed_weight, int64_t c_out, int64_t stride,
-                     const float * bias, int64_t padding, float * y, scratch ws, scratch pack, hipStream_t st) {
+                     const float * bias, int64_t padding, float * y, scratch_span ws, scratch_span pack, hipStream_t st) {
     return conv_transpose_entry(x, t, c_in, t, alpha_log, beta_log, param_type, packed_weight, c_out, stride, bias,
                                 padding, y, (t + 1) * stride - 2 * padding, ws.p, ws.floats, pack, st,
                                 "levo_hip_vae_decode");
@@ -1769,7 +1769,7 @@ extern "C" int levo_hip_snake_conv_transpose1d(const float * x, int64_t x_stride
                                                int64_t c_out, int64_t stride, const float * bias, int64_t padding,
                                                float * y, int64_t y_stride, levo_hip_stream_t stream) {
     return conv_transpose_entry(x, x_stride, c_in, t_in, alpha_log, beta_log, param_type, packed_weight, c_out,
-                                stride, bias, padding, y, y_stride, nullptr, 0, scratch{}, as_hip(stream),
+                                stride, bias, padding, y, y_stride, nullptr, 0, scratch_span{}, as_hip(stream),
                                 "levo_hip_snake_conv_transpose1d");
 }
 
@@ -1787,6 +1787,6 @@ extern "C" int levo_hip_snake_conv_transpose1d_split(const float * x, int64_t x_
                                                      int64_t padding, float * y, int64_t y_stride, float * workspace,
                                                      int64_t workspace_floats, levo_hip_stream_t stream) {
     return conv_transpose_entry(x, x_stride, c_in, t_in, alpha_log, beta_log, param_type, packed_weight, c_out,
-                                stride, bias, padding, y, y_stride, workspace, workspace_floats, scratch{}, as_hip(stream),
+                                stride, bias, padding, y, y_stride, workspace, workspace_floats, scratch_span{}, as_hip(stream),
                                 "levo_hip_snake_conv_transpose1d_split");
 }

@@ -70,9 +70,9 @@ bool weights_present(const levo_hip_vae_decoder_weights & w) { return missing_we
 
 // The free tail of a decoder buffer of n floats whose first `used` floats
 // hold a tensor: partial sums of the convolution that writes it.
-scratch tail_of(float * buf, int64_t n, int64_t used) {
+scratch_span tail_of(float * buf, int64_t n, int64_t used) {
     const int64_t start = (used + 63) / 64 * 64;  // 256-byte aligned
-    return start < n ? scratch{buf + start, n - start} : scratch{nullptr, 0};
+    return start < n ? scratch_span{buf + start, n - start} : scratch_span{nullptr, 0};
 }
 
 // run_residual (src/levo-vae.cpp:91-100); conv_0 writes h, conv_1 writes y.
@@ -84,12 +84,12 @@ scratch tail_of(float * buf, int64_t n, int64_t used) {
 // into pack_0 (the y buffer, which conv_1 writes) and the tail of h. The
 // public unit keeps h = conv_0's output.
 int residual_unit(const float * x, int64_t c, int64_t len, const levo_hip_vae_residual & u, int64_t dilation,
-                  levo_hip_type pt, float * y, float * h, bool post_in_h, scratch ws_h, scratch ws_y,
-                  scratch pack_0, scratch pack_h, levo_hip_stream_t stream) {
+                  levo_hip_type pt, float * y, float * h, bool post_in_h, scratch_span ws_h, scratch_span ws_y,
+                  scratch_span pack_0, scratch_span pack_h, levo_hip_stream_t stream) {
     const int fused = launch_residual_unit_fused(x, c, len, u.pre.alpha_log, u.pre.beta_log, u.conv_0.weight,
                                                  u.conv_0.bias, u.post.alpha_log, u.post.beta_log, u.conv_1.weight,
                                                  u.conv_1.bias, dilation, pt, y,
-                                                 post_in_h ? pack_h : scratch{}, as_hip(stream));
+                                                 post_in_h ? pack_h : scratch_span{}, as_hip(stream));
     if (fused != kNotFused) return fused;
     int st;
     if (!post_in_h) {
@@ -144,8 +144,8 @@ extern "C" int levo_hip_vae_residual_unit(const float * x, int64_t channels, int
     const uintptr_t yb = reinterpret_cast<uintptr_t>(y);
     const uintptr_t n = static_cast<uintptr_t>(channels * time) * sizeof(float);
     LEVO_REQUIRE(yb + n <= xb || xb + n <= yb, "vae_residual_unit: y must not overlap x");
-    return residual_unit(x, channels, time, *unit, dilation, param_type, y, h, false, scratch{},
-                         scratch{}, scratch{}, scratch{}, stream);
+    return residual_unit(x, channels, time, *unit, dilation, param_type, y, h, false, scratch_span{},
+                         scratch_span{}, scratch_span{}, scratch_span{}, stream);
 }
 
 extern "C" int levo_hip_vae_decode(const levo_hip_vae_decoder_weights * w, const float * latent, int64_t frames,
@@ -172,7 +172,7 @@ extern "C" int levo_hip_vae_decode(const levo_hip_vae_decoder_weights * w, const
     // input projection: no SnakeBeta in front (src/levo-vae.cpp:219-221)
     LEVO_STEP(decoder_conv1d(latent, kLatent, frames, nullptr, nullptr, pt, w->input.weight, kInWidth[0], 7,
                              w->input.bias, 3, 1, nullptr, a, nullptr, nullptr, tail_of(a, n, kInWidth[0] * frames),
-                             scratch{h, n}, as_hip(stream)));
+                             scratch_span{h, n}, as_hip(stream)));
     int64_t len = frames;
     for (int s = 0; s < 5; ++s) {
         const levo_hip_vae_stage & sg = w->stage[s];
@@ -180,8 +180,8 @@ extern "C" int levo_hip_vae_decode(const levo_hip_vae_decoder_weights * w, const
         const int64_t out_len = len * stride;  // (len + 1) s - 2 ((s + 1) / 2) for even s
         // b is the second third of the workspace here (each stage swaps a and b
         // four times), so its free tail and h are one piece
-        const scratch ws_up = tail_of(b, n, kOutWidth[s] * out_len);
-        const scratch pack = ws_up.p ? scratch{ws_up.p, ws_up.floats + n} : scratch{h, n};
+        const scratch_span ws_up = tail_of(b, n, kOutWidth[s] * out_len);
+        const scratch_span pack = ws_up.p ? scratch_span{ws_up.p, ws_up.floats + n} : scratch_span{h, n};
         LEVO_STEP(decoder_upsample(a, kInWidth[s], len, sg.activation.alpha_log, sg.activation.beta_log, pt,
                                    sg.upsample.weight, kOutWidth[s], stride, sg.upsample.bias, (stride + 1) / 2, b,
                                    ws_up, pack, as_hip(stream)));
@@ -191,7 +191,7 @@ extern "C" int levo_hip_vae_decode(const levo_hip_vae_decoder_weights * w, const
         // then the two swap
         for (int r = 0; r < 3; ++r) {
             LEVO_STEP(residual_unit(b, c, len, sg.residual[r], kDilations[r], pt, a, h, true, tail_of(h, n, c * len),
-                                    tail_of(a, n, c * len), scratch{a, n}, scratch{h, n}, stream));
+                                    tail_of(a, n, c * len), scratch_span{a, n}, scratch_span{h, n}, stream));
             std::swap(a, b);
         }
         if (stage_outputs != nullptr && stage_outputs[s] != nullptr) {
