@@ -37,7 +37,9 @@
 //
 // Infinities and NaN cannot be split (inf - inf): a workgroup whose inputs or
 // weights hold one (or a finite value that rounds to a bf16 infinity) redoes
-// its tile as plain F32 sums.
+// its tile as plain F32 sums. So does one with a sum that is not finite: where
+// a product passes the largest F32, its parts' products overflow apart, with
+// either sign, or only their first does.
 #include "conv_x3.hpp"
 
 #include "snake_math.hpp"
@@ -238,6 +240,14 @@ __device__ __forceinline__ void mfma_x3(const u32x4 (&a)[3], const u32x4 (&b)[2]
 // Row of accumulator item u of a 32 x 32 tile, in lane half hl.
 __device__ __forceinline__ int acc_row(int u, int hl) { return (u & 3) + 8 * (u >> 2) + 4 * hl; }
 
+// NaN when one of the sums is not finite.
+__device__ __forceinline__ float nonfinite_sums(const f32x16v & v) {
+    float bad = 0.0f;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) bad = __builtin_fmaf(v[u], 0.0f, bad);
+    return bad;
+}
+
 // The channel and phase of a row, its bias and output SnakeBeta, kept in LDS
 // for the epilogue.
 struct row_info {
@@ -376,6 +386,7 @@ __device__ __forceinline__ void unit_tail(const x3_kernel_params & p, u32x4 * ld
             const int64_t t = t0 + 64 * half + 32 * j + n;
             if (t >= c.cols) continue;
             out[j] = out[j] + lo[j];
+            bad += nonfinite_sums(out[j]);
 #pragma unroll
             for (int u = 0; u < 16; ++u) {
                 const int row = 32 * wave + acc_row(u, hl);
@@ -632,7 +643,11 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
 
     // ---- epilogue
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[j] = acc[j] + lo[j];
+    for (int j = 0; j < NJ; ++j) {
+        acc[j] = acc[j] + lo[j];
+        // k = 2 reads past what it stages for the columns it drops
+        if (32 * (j + 1) <= S::OUT || 32 * j + n < S::OUT) bad += nonfinite_sums(acc[j]);
+    }
     if constexpr (FUSE) {
         unit_tail(p, lds, acc, bad, t0);
     } else {

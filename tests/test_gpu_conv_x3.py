@@ -130,13 +130,56 @@ def test_values_that_cannot_be_split(hip, dev, oracle, kw, where):
         got, plain = (_run_t(hip, dev, x, w, b, 4, 2, split=s) for s in (True, False))
     else:
         got, plain = (_run(hip, dev, x, w, b, kw // 2, 1, ws_floats=n) for n in (-1, None))
+    _same_or_close(got, plain)
+
+
+def _direct_floats(c_in, rows, kw, cols):
+    """Workspace for the split weights and less than two partial sums: one split, the direct epilogue."""
+    pack = -(-rows // 32) * 32 * -(-c_in // 32) * 32 * kw * 3 // 2
+    return pack + pack // 64 + 8 * (c_in + rows) + 64 + rows * cols
+
+
+def _same_or_close(got, plain):
+    """The infinities and NaN of the F32 launch, its other values to F32 rounding at their size."""
     assert not np.all(np.isfinite(plain))
     assert np.array_equal(np.isnan(got), np.isnan(plain))
     inf = np.isinf(plain)
     assert np.array_equal(inf, np.isinf(got)) and np.array_equal(np.sign(got[inf]), np.sign(plain[inf]))
     ok = np.isfinite(plain)
-    # a sum with a 3.4e38 term is as large: relative to the value there
+    # a sum with a term of 3e38 is as large: relative to the value there
     assert np.max(np.abs(got[ok].astype(np.float64) - plain[ok]) / np.maximum(np.abs(plain[ok]), 1.0)) <= 2e-5
+
+
+# 2^64 (1 - 2^-10) squared is finite, the product of its bf16 roundings is not
+EDGE = np.float32(2.0 ** 64 * (1 - 2.0 ** -10))
+OVERFLOWS = [(1e30, -1e14), (1e30, 1e14), (1.003e25, 1.003e20), (-1e25, 1e20), (1.005e25, 1.001e20), (EDGE, EDGE)]
+
+
+@pytest.mark.parametrize("direct", [True, False])
+@pytest.mark.parametrize("kw", [7, 1, 3, 2])
+def test_products_that_overflow(hip, dev, oracle, kw, direct):
+    """Finite operands whose products pass the largest F32 (by far, where the
+    parts of the split operands overflow with either sign, and by so little that
+    only the product of their first parts does): the infinities, NaN and finite
+    values of the F32 launch, in one split and in several."""
+    c, c_out, t, stride = (256, 256, 20000, 1) if kw != 2 else (512, 256, 3000, 4)
+    if kw == 2:
+        x, w, b, _, _ = _t_case(oracle, c, c_out, t, stride, 31)
+    else:
+        x, w, b, _, _, _ = _case(oracle, c, c_out, t, kw, 31)
+    for i, (xv, wv) in enumerate(OVERFLOWS):
+        x[3 + 17 * i, 100 + 400 * i] = xv
+        if kw == 2:
+            w[3 + 17 * i, 5 + 40 * i, i] = wv
+        else:
+            w[5 + 40 * i, 3 + 17 * i, i % kw] = wv
+    n = _direct_floats(c, c_out * stride, kw, t + 1) if direct else -1
+    if kw == 2:
+        got, plain = _run_t(hip, dev, x, w, b, 4, 2, ws_floats=n), _run_t(hip, dev, x, w, b, 4, 2, split=False)
+    else:
+        got, plain = (_run(hip, dev, x, w, b, kw // 2, 1, ws_floats=m) for m in (n, None))
+    assert not np.array_equal(got[:, 3000:].view(np.uint32), plain[:, 3000:].view(np.uint32))  # the bf16 route
+    _same_or_close(got, plain)
 
 
 def _decode(hip, dev, dw, latent, frames, stage5):
@@ -174,3 +217,24 @@ def test_unit_with_a_weight_that_cannot_be_split(hip, binding, dev, oracle):
     others = np.arange(128) != row
     assert f32_err(after[others], before[others]) <= 1e-5
     assert not np.any(np.isnan(after)) and np.mean(np.abs(after[row]) > 1e30) > 0.99
+
+
+def test_unit_with_products_that_overflow(hip, binding, dev, oracle):
+    """1e25 in a channel between the last unit's convolutions, 1e20 against it in
+    a row of the k = 1 weights: that row is infinite, with the sign of the
+    product, the other rows stay within F32 rounding of 1e25 times their weight."""
+    frames, row = 7, 11
+    w = Weights(binding, 61)
+    latent = oracle.gaussian(64 * frames, 9).reshape(64, frames)
+    unit = w.stages[4]["res"][2]
+    unit["conv0"][1][5] = np.float32(1.0037e25)
+    dw, keep = device_weights(hip, binding, dev, w)
+    before = _decode(hip, dev, dw, latent, frames, True)
+    assert np.all(np.isfinite(before))
+    for sign in (1, -1):
+        unit["conv1"][0][row, 5, 0] = np.float32(sign * 1.0021e20)
+        dw, keep = device_weights(hip, binding, dev, w)
+        after = _decode(hip, dev, dw, latent, frames, True)
+        assert np.all(np.isinf(after[row])) and np.all(np.sign(after[row]) == sign)
+        others = np.arange(128) != row
+        assert f32_err(after[others], before[others]) <= 1e-5

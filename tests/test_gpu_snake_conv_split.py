@@ -186,7 +186,7 @@ def test_rejects_bad_workspace(hip, dev, binding):
 
 # ---- transposed convolution (levo_hip_snake_conv_transpose1d_split) --------
 
-def _run_t(hip, dev, x, w, b, stride, pad, a=None, bl=None, param_type=0, split=True):
+def _run_t(hip, dev, x, w, b, stride, pad, a=None, bl=None, param_type=0, split=True, ws_floats=-1):
     import torch
     c_in, t_in = x.shape
     _, c_out, _ = w.shape
@@ -198,7 +198,7 @@ def _run_t(hip, dev, x, w, b, stride, pad, a=None, bl=None, param_type=0, split=
                   beta_log=to_dev(bl, dev) if bl is not None else None, param_type=param_type,
                   bias=to_dev(b, dev) if b is not None else None, padding=pad, y=y)
     if split:
-        n = hip.snake_conv_transpose1d_split_workspace_floats(c_out, t_in, stride)
+        n = hip.snake_conv_transpose1d_split_workspace_floats(c_out, t_in, stride) if ws_floats < 0 else ws_floats
         ws = torch.full((n,), float("nan"), dtype=torch.float32, device=dev)
         hip.snake_conv_transpose1d_split(to_dev(x, dev), c_in, t_in, packed, c_out, stride, workspace=ws,
                                          workspace_floats=n, **kwargs)
