@@ -35,11 +35,16 @@
 //   per workgroup: 0.94 of the speed; one wave a SIMD with 64 x 128: 0.87; four
 //   waves a workgroup, two workgroups a CU (twice the staging): 0.92.
 //
-// Infinities and NaN cannot be split (inf - inf): a workgroup whose inputs or
-// weights hold one (or a finite value that rounds to a bf16 infinity) redoes
-// its tile as plain F32 sums. So does one with a sum that is not finite: where
-// a product passes the largest F32, its parts' products overflow apart, with
-// either sign, or only their first does.
+// Infinities and NaN: the first part carries them, the others are NaN then. The
+// hi hi sums have accumulators of their own, so where one is not finite it is
+// the output as it stands: an infinite or NaN operand makes it what the F32 sum
+// is, and what the small products did does not matter (a decode of 252 frames, all
+// of it NaN in the end: 10.7 ms with the look through the tiles' inputs, 7.2 ms for
+// an ordinary one; F32 launches 16 and 13.5 ms). What that does not cover
+// is summed again in plain F32, by the workgroup whose tile it is (f32_needed):
+// sums that are not finite where a finite product may overflow (its parts'
+// products overflow apart, or only the first does) or an operand is so small
+// that its first part may be zero. 20 to 40 times the tile's time.
 #include "conv_x3.hpp"
 
 #include "snake_math.hpp"
@@ -55,6 +60,8 @@ constexpr int kUnit = 128;  // channels of a fused residual unit
 constexpr int kCI = 16;     // input channels per K step
 constexpr int kMaxHalo = 64;  // (taps - 1) * dilation: k = 7 up to dilation 10
 constexpr int kNT = 128;      // columns per workgroup
+constexpr int kUnitItems = 6 * (kUnit / kCI) * 64;  // half a unit's h: [16 channels][plane][8 channels][column]
+constexpr int kUnitInfoItems = kUnit * 24 / 16;     // unit_row per channel
 
 template <int KW, bool FUSE>
 struct x3_shape {
@@ -74,6 +81,10 @@ struct x3_shape {
     // Pairs of channels staged per thread and chunk: main columns, then halo.
     static constexpr int MAIN = 16 * CG / WAVES;
     static constexpr int PAIRS = MAIN + (HALO ? 8 / WAVES : 0);
+    // LDS: two buffers of a chunk, over them what the epilogue needs; then the
+    // words of tile_state
+    static constexpr int STATE = FUSE ? std::max(2 * BUF, kUnitItems + kUnitInfoItems) : 2 * BUF;
+    static constexpr int LDS_ITEMS = STATE + 2;
 };
 
 typedef float f32x2v __attribute__((ext_vector_type(2)));
@@ -86,7 +97,7 @@ typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
 struct x3_kernel_params {
     x3_conv c;
     const u32x4 * w;         // packed fragments
-    const uint32_t * w_bad;  // [32-row tiles][channel groups]: the weights hold a value that cannot be split
+    const uint32_t * w_range;  // [32-row tiles][channel groups]: value_range of the weights
     const snake_param * pre;   // [channel groups * 16] (c.snake)
     const snake_param * post;  // [c_out] (c.post_alpha_log)
     int32_t rows;            // c_out * stride
@@ -97,7 +108,7 @@ struct x3_kernel_params {
     int64_t part_slice, part_pitch;
     // the k = 1 convolution of a residual unit (unit_tail)
     const u32x4 * w1;
-    const uint32_t * w1_bad;
+    const uint32_t * w1_range;
     const float * w1_raw;
     const float * bias1;
 };
@@ -106,15 +117,12 @@ __device__ __forceinline__ uint32_t pack2(bf16x2 v) { return __builtin_bit_cast(
 __device__ __forceinline__ float lo_f32(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
 __device__ __forceinline__ float hi_f32(uint32_t v) { return __builtin_bit_cast(float, v & 0xffff0000u); }
 
-// Two values into their three bf16 parts. `bad` turns NaN when a part is not
-// finite.
-__device__ __forceinline__ void split2(float a, float b, uint32_t (&o)[3], float & bad) {
+// Two values into their three bf16 parts. An infinity or NaN is its first part,
+// the other two are NaN.
+__device__ __forceinline__ void split2(float a, float b, uint32_t (&o)[3]) {
     o[0] = pack2(__builtin_convertvector(f32x2v{a, b}, bf16x2));
-    const float ah = lo_f32(o[0]), bh = hi_f32(o[0]);
-    bad = __builtin_fmaf(ah, 0.0f, bad);
-    bad = __builtin_fmaf(bh, 0.0f, bad);
-    a -= ah;
-    b -= bh;
+    a -= lo_f32(o[0]);
+    b -= hi_f32(o[0]);
     o[1] = pack2(__builtin_convertvector(f32x2v{a, b}, bf16x2));
     a -= lo_f32(o[1]);
     b -= hi_f32(o[1]);
@@ -122,15 +130,37 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t (&o)[3], float
 }
 
 template <int N>
-__device__ __forceinline__ void split_n(const float (&v)[N], uint32_t (&o)[3][N / 2], float & bad) {
+__device__ __forceinline__ void split_n(const float (&v)[N], uint32_t (&o)[3][N / 2]) {
 #pragma unroll
     for (int i = 0; i < N / 2; ++i) {
         uint32_t t[3];
-        split2(v[2 * i], v[2 * i + 1], t, bad);
+        split2(v[2 * i], v[2 * i + 1], t);
         o[0][i] = t[0];
         o[1][i] = t[1];
         o[2][i] = t[2];
     }
+}
+
+// The range of some values: the bits of the largest finite |v|, with kHasTiny
+// where a value other than zero is below 2^-100.
+constexpr uint32_t kHasTiny = 0x80000000u;
+constexpr uint32_t kInfBits = 0x7f800000u;
+constexpr float kTinyBelow = 0x1p-100f;
+
+__device__ __forceinline__ uint32_t join_ranges(uint32_t a, uint32_t b) {
+    return std::max(a & ~kHasTiny, b & ~kHasTiny) | ((a | b) & kHasTiny);
+}
+
+__device__ __forceinline__ uint32_t value_range(float v) {
+    const float m = __builtin_fabsf(v);
+    const uint32_t b = __builtin_bit_cast(uint32_t, m);
+    return b >= kInfBits ? 0 : b | (m != 0.0f && m < kTinyBelow ? kHasTiny : 0);
+}
+
+__device__ __forceinline__ uint32_t wave_range(uint32_t r) {
+#pragma unroll
+    for (int n = 32; n >= 1; n >>= 1) r = join_ranges(r, __shfl_xor(r, n));
+    return r;
 }
 
 __device__ __forceinline__ float param_at(const void * p, int32_t f16, int i) {
@@ -156,23 +186,27 @@ __device__ __forceinline__ snake_param scalar_param(const snake_param * p, int i
 // weights, three 16-byte stores. The blocks after the last one evaluate SnakeBeta parameters.
 // With w1 (a residual unit's k = 1 weights, 128 x 128) KW of its (32-row tile,
 // 16-channel group) pairs are a block's.
-__device__ __forceinline__ bool pack_item(const float * src, int ci_left, int ci_step, u32x4 * dst, int lane) {
+// Returns the range of the lane's weights.
+__device__ __forceinline__ uint32_t pack_item(const float * src, int ci_left, int ci_step, u32x4 * dst, int lane) {
     float v[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) v[i] = i < ci_left ? src[i * ci_step] : 0.0f;
     uint32_t o[3][4];
-    float bad = 0.0f;
-    split_n<8>(v, o, bad);
+    split_n<8>(v, o);
 #pragma unroll
     for (int p = 0; p < 3; ++p) dst[64 * p + lane] = u32x4{o[p][0], o[p][1], o[p][2], o[p][3]};
-    return bad != 0.0f;
+    uint32_t range = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) range = join_ranges(range, value_range(v[i]));
+    return range;
 }
 
 template <int KW>
-__global__ __launch_bounds__(64 * KW) void x3_pack_kernel(const x3_conv c, u32x4 * w, uint32_t * w_bad,
+__global__ __launch_bounds__(64 * KW) void x3_pack_kernel(const x3_conv c, u32x4 * w, uint32_t * w_range,
                                                           snake_param * pre, snake_param * post, int rows, int groups,
                                                           int row_tiles, const float * w1, u32x4 * w1_packed,
-                                                          uint32_t * w1_bad) {
+                                                          uint32_t * w1_range) {
+    __shared__ uint32_t tap_range[KW];
     int b = static_cast<int>(blockIdx.x);
     const int tid = static_cast<int>(threadIdx.x);
     const int tap = tid >> 6;
@@ -183,9 +217,16 @@ __global__ __launch_bounds__(64 * KW) void x3_pack_kernel(const x3_conv c, u32x4
         const int ci = (b - rt * groups) * kCI + 8 * (lane >> 5);
         const int co = row / c.stride;
         const float * src = c.w + ((static_cast<int64_t>(row - co * c.stride) * c.c_out + co) * c.c_in + ci) * KW + tap;
-        const bool bad = pack_item(src, row < rows ? c.c_in - ci : 0, KW, w + (static_cast<int64_t>(b) * KW + tap) * 192, lane);
-        const int any = __syncthreads_or(bad);
-        if (tid == 0) w_bad[b] = static_cast<uint32_t>(any);
+        const uint32_t range =
+                wave_range(pack_item(src, row < rows ? c.c_in - ci : 0, KW, w + (static_cast<int64_t>(b) * KW + tap) * 192, lane));
+        if (lane == 0) tap_range[tap] = range;
+        __syncthreads();
+        if (tid == 0) {
+            uint32_t all = 0;
+#pragma unroll
+            for (int k = 0; k < KW; ++k) all = join_ranges(all, tap_range[k]);
+            w_range[b] = all;
+        }
         return;
     }
     b -= row_tiles * groups;
@@ -196,9 +237,14 @@ __global__ __launch_bounds__(64 * KW) void x3_pack_kernel(const x3_conv c, u32x4
             if (item >= kItems) return;
             const int row = item / (kUnit / kCI) * 32 + (lane & 31);
             const int ci = item % (kUnit / kCI) * kCI + 8 * (lane >> 5);
-            const bool bad = pack_item(w1 + row * kUnit + ci, 8, 1, w1_packed + item * 192, lane);
-            const bool any = __ballot(bad) != 0;
-            if (lane == 0) w1_bad[item] = any;
+            const float * src = w1 + row * kUnit + ci;
+            uint32_t range = wave_range(pack_item(src, 8, 1, w1_packed + item * 192, lane));
+            // one that is not finite counts as the largest here: the tiles are summed in F32
+            bool finite = true;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) finite &= __builtin_fabsf(src[i]) < __builtin_inff();
+            if (__ballot(!finite) != 0) range = kInfBits;
+            if (lane == 0) w1_range[item] = range;
             return;
         }
         b -= (kItems + KW - 1) / KW;
@@ -240,12 +286,37 @@ __device__ __forceinline__ void mfma_x3(const u32x4 (&a)[3], const u32x4 (&b)[2]
 // Row of accumulator item u of a 32 x 32 tile, in lane half hl.
 __device__ __forceinline__ int acc_row(int u, int hl) { return (u & 3) + 8 * (u >> 2) + 4 * hl; }
 
-// NaN when one of the sums is not finite.
-__device__ __forceinline__ float nonfinite_sums(const f32x16v & v) {
-    float bad = 0.0f;
+// acc += lo; where acc, the sum of the products of the operands' first parts,
+// is not finite it is the sum as it stands. `bad` turns NaN where a sum is not
+// finite.
+__device__ __forceinline__ void join_sums(f32x16v & acc, const f32x16v & lo, float & bad) {
 #pragma unroll
-    for (int u = 0; u < 16; ++u) bad = __builtin_fmaf(v[u], 0.0f, bad);
-    return bad;
+    for (int u = 0; u < 16; ++u) {
+        const float sum = acc[u] + lo[u];
+        acc[u] = __builtin_fabsf(acc[u]) < __builtin_inff() ? sum : acc[u];
+        bad = __builtin_fmaf(acc[u], 0.0f, bad);
+    }
+}
+
+// What a workgroup has seen; each wave's go into tile_state::seen.
+enum : uint32_t { kSumNotFinite = 1 };
+
+struct tile_state {
+    uint32_t seen;
+    // ranges over the tile (f32_needed)
+    uint32_t w, x_bound, x_infinite;
+    uint32_t mid, w1;
+    uint32_t pad[2];
+};
+static_assert(sizeof(tile_state) == 32, "two items of LDS");
+
+__device__ __forceinline__ uint32_t seen_if(bool lane_has, uint32_t bit) { return __ballot(lane_has) != 0 ? bit : 0; }
+
+__device__ __forceinline__ bool worth_a_look(uint32_t seen) { return (seen & kSumNotFinite) != 0; }
+
+// Whether sums of n products of values up to a and b may overflow.
+__device__ __forceinline__ bool out_of_split_range(float a, float b, float n) {
+    return a >= 0x1p126f || b >= 0x1p126f || a * b * n >= 0x1p126f;
 }
 
 // The channel and phase of a row, its bias and output SnakeBeta, kept in LDS
@@ -292,27 +363,73 @@ __device__ __forceinline__ void plain_sums(const x3_kernel_params & p, int row, 
     }
 }
 
+// Whether a tile worth a look has to be summed in plain F32: looks through its
+// inputs (columns col0 .. of kNT and the halo; SnakeBeta adds up to 1 / beta)
+// and the ranges of its weights. Every thread of the workgroup calls it and
+// gets the same answer.
+template <int KW, int THREADS>
+__device__ __forceinline__ bool f32_needed(const x3_kernel_params & p, tile_state * state, int rt0, int row_tiles,
+                                           int64_t col0, int chunk0, int chunk1) {
+    constexpr int CG = KW <= 2 ? 2 : 1;
+    const x3_conv & c = p.c;
+    const int tid = static_cast<int>(threadIdx.x);
+    uint32_t wr = 0;
+    for (int e = tid; e < row_tiles * (chunk1 - chunk0) * CG; e += THREADS) {
+        const int rt = rt0 + e % row_tiles;
+        if (rt * 32 < p.rows) wr = join_ranges(wr, p.w_range[rt * p.chunks * CG + chunk0 * CG + e / row_tiles]);
+    }
+    uint32_t xr = 0, infinite = 0;
+    float bound = 0.0f;
+    const int span = kNT + (KW - 1) * c.dil;
+    const int ci0 = chunk0 * kCI * CG, ci1 = std::min(chunk1 * kCI * CG, c.c_in);
+#pragma unroll 1
+    for (int col = tid % 64; col < span; col += 64) {
+        const int64_t t = col0 - c.pad + col;
+        if (t < 0 || t >= c.t_in) continue;
+#pragma unroll 4
+        for (int ci = ci0 + tid / 64; ci < ci1; ci += THREADS / 64) {
+            const float v = __builtin_fabsf(c.x[ci * c.x_pitch + t]);
+            xr = join_ranges(xr, value_range(v));
+            infinite |= v == __builtin_inff();
+            const float b = c.snake ? v + __builtin_fmaxf(p.pre[ci].rbeta, 0.0f) : v;
+            if (v < __builtin_inff()) bound = __builtin_fmaxf(bound, b);
+        }
+    }
+    atomicMax(&state->w, wr & ~kHasTiny);
+    atomicMax(&state->x_bound, __builtin_bit_cast(uint32_t, bound));
+    atomicOr(&state->x_infinite, (infinite ? 1u : 0u) | (xr & kHasTiny ? 2u : 0u) | (wr & kHasTiny ? 4u : 0u));
+    __syncthreads();
+    const uint32_t odd = state->x_infinite;
+    // an infinity times a value whose first part may be zero (one of the weights
+    // times a tiny input, or the other way)
+    if ((state->seen & kSumNotFinite) && ((odd & 2) || (odd & 5) == 5)) return true;
+    return out_of_split_range(__builtin_bit_cast(float, state->x_bound), __builtin_bit_cast(float, state->w),
+                              static_cast<float>((ci1 - ci0) * KW));
+}
+
 // The k = 1 half of a residual unit of 128 channels, in the k = 7 launch: a
 // workgroup holds every channel of its 128 columns. h = acc + bias goes through
 // the post SnakeBeta, split, into LDS (in two halves of 64 columns, so that two
 // workgroups share a CU) as the B operand of the k = 1 weights, which come from
-// L2 like the others; the result + bias + the unit's input is the output. `bad`
-// from the first convolution, or of an h that cannot be split, redoes the tile.
+// L2 like the others; the result + bias + the unit's input is the output. A tile
+// whose sums or operands ask for it (f32_needed, the same for h and the k = 1
+// weights) is summed again in plain F32 over what was stored.
 struct unit_row {
     float bias0, bias1;
     snake_param post;
     float pad;
 };
-constexpr int kUnitItems = 6 * (kUnit / kCI) * 64;  // [16 channels][plane][8 channels][column]
+static_assert(sizeof(unit_row) * kUnit == kUnitInfoItems * 16, "unit_row fills its items");
 
 __device__ __forceinline__ void unit_tail(const x3_kernel_params & p, u32x4 * lds, const f32x16v (&acc)[kNT / 32],
-                                          float bad, int64_t t0) {
+                                          tile_state * state, uint32_t seen, int64_t t0) {
     const x3_conv & c = p.c;
     const int tid = static_cast<int>(threadIdx.x);
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 31;
     const int hl = lane >> 5;
+    float bad = 0.0f, largest = 0.0f;
     unit_row * info = reinterpret_cast<unit_row *>(lds + kUnitItems);
     if (tid < kUnit) info[tid] = unit_row{c.bias ? c.bias[tid] : 0.0f, p.bias1 ? p.bias1[tid] : 0.0f, p.post[tid], 0.0f};
     const char * wp = reinterpret_cast<const char *>(p.w1) + static_cast<int64_t>(wave) * (kUnit / kCI) * 3072;
@@ -330,7 +447,7 @@ __device__ __forceinline__ void unit_tail(const x3_kernel_params & p, u32x4 * ld
 #pragma unroll
         for (int s = 0; s < 3; ++s) a[0][s] = *reinterpret_cast<const u32x4 *>(wp + 16 * lane + 1024 * s);
         __syncthreads();  // info is there; the first half's fragments are read
-        auto store_h = [&](bool exact, bool & slow, float & nonfinite) __attribute__((always_inline)) {
+        auto store_h = [&](bool exact, bool & slow) __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -343,8 +460,10 @@ __device__ __forceinline__ void unit_tail(const x3_kernel_params & p, u32x4 * ld
                         if (c.bias) h = h + ri.bias0;
                         v[q] = exact ? snake(h, ri.post) : snake_fast(h, ri.post, slow);
                     }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) largest = __builtin_fmaxf(largest, __builtin_fabsf(v[q]));
                     uint32_t o[3][2];
-                    split_n<4>(v, o, nonfinite);
+                    split_n<4>(v, o);
                     // rows 32 wave + 8 (u / 4) + 4 hl ..: half an item of channel group row / 8
                     const int item = (2 * wave + u / 8) * 6 * 64 + ((u >> 2) & 1) * 64 + 32 * j + n;
 #pragma unroll
@@ -353,13 +472,12 @@ __device__ __forceinline__ void unit_tail(const x3_kernel_params & p, u32x4 * ld
                 }
         };
         bool slow = false;
-        float nonfinite = 0.0f;
-        store_h(false, slow, nonfinite);
+        const float before = largest;
+        store_h(false, slow);
         if (slow) {  // rare: arguments beyond the reduced sine's range
-            nonfinite = 0.0f;
-            store_h(true, slow, nonfinite);
+            largest = before;
+            store_h(true, slow);
         }
-        bad += nonfinite;
         __syncthreads();
         f32x16v out[2], lo[2];
 #pragma unroll
@@ -385,8 +503,7 @@ __device__ __forceinline__ void unit_tail(const x3_kernel_params & p, u32x4 * ld
         for (int j = 0; j < 2; ++j) {
             const int64_t t = t0 + 64 * half + 32 * j + n;
             if (t >= c.cols) continue;
-            out[j] = out[j] + lo[j];
-            bad += nonfinite_sums(out[j]);
+            join_sums(out[j], lo[j], bad);
 #pragma unroll
             for (int u = 0; u < 16; ++u) {
                 const int row = 32 * wave + acc_row(u, hl);
@@ -398,7 +515,15 @@ __device__ __forceinline__ void unit_tail(const x3_kernel_params & p, u32x4 * ld
     };
     run_half(std::integral_constant<int, 0>{});
     run_half(std::integral_constant<int, 1>{});
-    if (!__syncthreads_or(bad != 0.0f)) return;
+    seen |= seen_if(bad != 0.0f, kSumNotFinite);
+    if (lane == 0) atomicOr(&state->seen, seen);
+    __syncthreads();
+    if (!worth_a_look(state->seen)) return;
+    atomicMax(&state->mid, __builtin_bit_cast(uint32_t, largest));
+    if (tid < kUnit / 32 * (kUnit / kCI)) atomicMax(&state->w1, p.w1_range[tid] & ~kHasTiny);
+    if (!f32_needed<7, kThreads>(p, state, 0, kUnit / 32, t0, 0, p.chunks) &&
+        !out_of_split_range(__builtin_bit_cast(float, state->mid), __builtin_bit_cast(float, state->w1), kUnit))
+        return;
     // plain F32, 32 columns of h at a time
     float * hs = reinterpret_cast<float *>(lds);
 #pragma unroll 1
@@ -453,19 +578,9 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
     const int n = lane & 31;
     const int hl = lane >> 5;
 
-    float bad = 0.0f;
-    {
-        // weights of this workgroup that cannot be split
-        uint32_t wb = 0;
-        const int g_begin = c_begin * S::CG;
-        const int n_flags = S::WAVES * (c_end - c_begin) * S::CG;
-        for (int e = tid; e < n_flags; e += S::THREADS) {
-            const int rt = row0 / 32 + e % S::WAVES;
-            if (rt * 32 < p.rows) wb |= p.w_bad[rt * p.chunks * S::CG + g_begin + e / S::WAVES];
-        }
-        if (FUSE && tid < kUnit / 32 * (kUnit / kCI)) wb |= p.w1_bad[tid];
-        if (wb) bad = __builtin_nanf("");
-    }
+    tile_state * state = reinterpret_cast<tile_state *>(lds + S::STATE);
+    if (tid < static_cast<int>(sizeof(tile_state) / 4)) reinterpret_cast<uint32_t *>(state)[tid] = 0;
+    uint32_t seen = 0;  // the wave's
 
     // Staging: waves deal the columns, channel halves and groups of a chunk
     // among them, in pairs of channels; the eight channels of a column's item
@@ -505,8 +620,8 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
     };
     // Pair m through SnakeBeta, in three planes; the second of two neighbouring
     // pairs stores both pairs' eight bytes in each plane.
-    auto stage_pair = [&](int chunk, int buf, int m, bool exact, uint32_t (&o)[3][2], bool & slow,
-                          float & nonfinite) __attribute__((always_inline)) {
+    auto stage_pair = [&](int chunk, int buf, int m, bool exact, uint32_t (&o)[3][2],
+                          bool & slow) __attribute__((always_inline)) {
         int u, col, ch;
         pair_place(m, lane, u, col, ch);
         const int ci = chunk * S::CI + 16 * u + 8 * kg + ch;
@@ -522,7 +637,7 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
             }
         }
         uint32_t w[3];
-        split2(v[0], v[1], w, nonfinite);
+        split2(v[0], v[1], w);
         u32x4 * item = lds + buf * S::BUF + u * S::GROUP + kg * S::W + col;
         if (S::WAVES == 8 && m >= S::MAIN) {  // a single halo pair
 #pragma unroll
@@ -540,7 +655,7 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
         uint32_t o[3][2];
         bool slow = false;
 #pragma unroll
-        for (int m = 0; m < S::PAIRS; ++m) stage_pair(chunk, buf, m, true, o, slow, bad);
+        for (int m = 0; m < S::PAIRS; ++m) stage_pair(chunk, buf, m, true, o, slow);
     };
 
     // weight fragments: rows 32 * wave of the tile; a K step is 3072 bytes
@@ -600,7 +715,6 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
             u32x4 b[2][2][3];
             uint32_t o[3][2];
             bool slow = false;
-            float nonfinite = 0.0f;
 #pragma unroll
             for (int s = 0; s < 6; ++s) b[0][s / 3][s % 3] = bp[(s % 3) * 2 * S::W + 32 * (s / 3)];
 #pragma unroll
@@ -625,7 +739,7 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
                 if (g >= kFirst) {
                     const int m0 = (g - kFirst) * kPairs / kSpan, m1 = (g + 1 - kFirst) * kPairs / kSpan;
 #pragma unroll
-                    for (int m = m0; m < m1; ++m) stage_pair(next, buf ^ 1, m, false, o, slow, nonfinite);
+                    for (int m = m0; m < m1; ++m) stage_pair(next, buf ^ 1, m, false, o, slow);
 #pragma unroll
                     for (int q = 0; q < 12; ++q) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -636,20 +750,24 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
             }
             step += S::KS;
             if (SNAKE && slow) stage_all(next, buf ^ 1);  // rare: arguments beyond the reduced sine's range
-            else bad += nonfinite;
             __syncthreads();
         }
     }
 
     // ---- epilogue
+    {
+        float bad = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        acc[j] = acc[j] + lo[j];
-        // k = 2 reads past what it stages for the columns it drops
-        if (32 * (j + 1) <= S::OUT || 32 * j + n < S::OUT) bad += nonfinite_sums(acc[j]);
+        for (int j = 0; j < NJ; ++j) {
+            // k = 2 reads past what it stages for the columns it drops
+            float tile_bad = 0.0f;
+            join_sums(acc[j], lo[j], tile_bad);
+            if (32 * (j + 1) <= S::OUT || 32 * j + n < S::OUT) bad += tile_bad;
+        }
+        seen = seen_if(bad != 0.0f, kSumNotFinite);
     }
     if constexpr (FUSE) {
-        unit_tail(p, lds, acc, bad, t0);
+        unit_tail(p, lds, acc, state, seen, t0);
     } else {
         // every residual load before any store (y may be the residual), and all
         // of them at once: one trip to memory (clamped, masked at the store)
@@ -665,7 +783,10 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
             }
         }
         row_info * info = reinterpret_cast<row_info *>(lds);
-        const int redo = __syncthreads_or(bad != 0.0f);
+        if (lane == 0) atomicOr(&state->seen, seen);
+        __syncthreads();
+        const bool redo = worth_a_look(state->seen) &&
+                          f32_needed<KW, S::THREADS>(p, state, row0 / 32, S::WAVES, t0, c_begin, c_end);
         if (tid < S::ROWS) {
             const int row = std::min(row0 + tid, p.rows - 1);
             row_info ri{};
@@ -876,8 +997,8 @@ int pick_splits(const x3_conv & c, const x3_layout & l, int64_t tiles, int64_t k
 template <int KW, bool SNAKE, bool FUSE>
 int launch_kernel(const x3_kernel_params & p, hipStream_t st, const char * what) {
     using S = x3_shape<KW, FUSE>;
-    const size_t lds = std::max({2 * sizeof(u32x4) * S::BUF, S::ROWS * sizeof(row_info),
-                                 FUSE ? sizeof(u32x4) * kUnitItems + kUnit * sizeof(unit_row) : size_t{0}});
+    static_assert(S::ROWS * sizeof(row_info) <= sizeof(u32x4) * S::STATE, "the epilogue's rows fit the buffers");
+    const size_t lds = sizeof(u32x4) * S::LDS_ITEMS;
     const void * fn = reinterpret_cast<const void *>(&x3_conv_kernel<KW, SNAKE, FUSE>);
     if (const int rc = allow_dynamic_lds(fn, 80 * 1024, what); rc != LEVO_HIP_OK) return rc;
     const uint32_t grid = static_cast<uint32_t>(ceil_div(p.tiles, 8) * 8 * p.splits);
@@ -897,13 +1018,13 @@ int launch_pack(x3_kernel_params & p, const x3_conv & c, const x3_layout & l, ch
     u32x4 * frag1 = reinterpret_cast<u32x4 *>(pack += l.post_bytes);
     uint32_t * flags1 = reinterpret_cast<uint32_t *>(pack + kUnitFragBytes);
     p.w = frag;
-    p.w_bad = flags;
+    p.w_range = flags;
     p.pre = pre;
     p.post = post;
     p.rows = static_cast<int32_t>(l.rows);
     p.chunks = static_cast<int32_t>(l.chunks);
     p.w1 = frag1;
-    p.w1_bad = flags1;
+    p.w1_range = flags1;
     p.w1_raw = w1;
     const int64_t tx = ceil_div(c.cols, x3_shape<KW, FUSE>::OUT);
     p.tiles_x = static_cast<int32_t>(tx);

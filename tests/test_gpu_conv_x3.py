@@ -238,3 +238,86 @@ def test_unit_with_products_that_overflow(hip, binding, dev, oracle):
         assert np.all(np.isinf(after[row])) and np.all(np.sign(after[row]) == sign)
         others = np.arange(128) != row
         assert f32_err(after[others], before[others]) <= 1e-5
+
+
+def _last_stage(hip, binding, dev, w, dw, latent, frames):
+    """Stage 5 as the decode computes it (one-launch bf16 units), and from the
+    decode's stage 4 output by the public upsampler and residual units (F32)."""
+    import torch
+    nbytes = hip.vae_decode_workspace_bytes(frames)
+    ws = torch.full((nbytes // 4,), float("nan"), device=dev)
+    audio = torch.empty(2, 1920 * frames, device=dev)
+    s4, s5 = torch.empty(128, 960 * frames, device=dev), torch.empty(128, 1920 * frames, device=dev)
+    hip.vae_decode(dw, to_dev(latent, dev), frames, audio, ws, nbytes, stage_outputs=[None] * 3 + [s4, s5])
+    stage = dw.stage[4]
+    x, y, h = (torch.empty(128, 1920 * frames, device=dev) for _ in range(3))
+    hip.snake_conv_transpose1d(s4, 128, 960 * frames, stage.upsample.weight, 128, 2,
+                               alpha_log=stage.activation.alpha_log, beta_log=stage.activation.beta_log,
+                               bias=stage.upsample.bias, padding=1, y=x)
+    for unit, dil in zip(stage.residual, (1, 3, 9)):
+        hip.vae_residual_unit(x, 128, 1920 * frames, unit, dil, y, h)
+        x, y = y, x
+    torch.cuda.synchronize()
+    return from_dev(s5), from_dev(x)
+
+
+@pytest.mark.parametrize("what", ["x nan", "h inf", "h large", "x large", "w0 inf", "w0 nan", "w0 3.4e38", "w1 inf", "w1 nan"])
+def test_unit_special_values(hip, binding, dev, oracle, what):
+    """A NaN in the latent, infinite and very large (sine arguments beyond the
+    reduced form's) inputs and inner values, weights that are not finite: the
+    infinities and NaN of the F32 units, the other values to their rounding."""
+    frames = 9
+    w = Weights(binding, 70)
+    latent = oracle.gaussian(64 * frames, 11).reshape(64, frames)
+    unit = w.stages[4]["res"][1]
+    where, value = what.split()
+    if what == "x nan":
+        w.stages[4]["res"][0]["conv1"][1][3] = np.nan  # a channel of the second unit's input
+    elif what == "x large":
+        w.stages[4]["res"][0]["conv1"][1][::9] = np.float32(3e4)
+        unit["conv0"][0][:, ::9] *= np.float32(1e-4)
+    elif where == "h":
+        unit["conv0"][1][::9] = np.float32({"inf": np.inf, "large": 3e4}[value])
+        unit["conv1"][0][:, ::9] *= np.float32(1e-4)
+    else:
+        unit["conv" + where[1]][0][17, 5, 0] = np.float32(value)
+    dw, keep = device_weights(hip, binding, dev, w)
+    got, plain = _last_stage(hip, binding, dev, w, dw, latent, frames)
+    nan = np.isnan(plain)
+    assert np.array_equal(np.isnan(got), nan)
+    inf = np.isinf(plain)
+    assert np.array_equal(np.isinf(got), inf) and np.array_equal(np.sign(got[inf]), np.sign(plain[inf]))
+    assert np.any(nan | inf) == (value not in ("large", "3.4e38"))
+    ok = np.isfinite(plain)
+    if np.any(ok):
+        # two F32 sums of 896 and 128 terms, three units: at the scale of their terms
+        scale = {"large": 3e4, "3.4e38": np.max(np.abs(plain[ok]))}.get(value, np.maximum(np.abs(plain[ok]), 1.0))
+        assert np.max(np.abs(got[ok].astype(np.float64) - plain[ok]) / scale) <= 2e-5
+
+
+def test_nan_costs_no_more_than_numbers(hip, binding, dev, oracle):
+    """A decode of a latent with a NaN (in the end all of the audio): within twice
+    the time of an ordinary one, as the F32 launches took the same for both."""
+    import torch
+    frames = 64
+    w = Weights(binding, 80)
+    dw, keep = device_weights(hip, binding, dev, w)
+    nbytes = hip.vae_decode_workspace_bytes(frames)
+    ws = torch.empty(nbytes // 4, device=dev)
+    audio = torch.empty(2, 1920 * frames, device=dev)
+    latent = to_dev(oracle.gaussian(64 * frames, 12).reshape(64, frames), dev)
+    odd = latent.clone()
+    odd[7, 5::11] = float("nan")
+    times = {}
+    for name, x in (("numbers", latent), ("nan", odd)):
+        best = 1e9
+        for _ in range(4):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            hip.vae_decode(dw, x, frames, audio, ws, nbytes)
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        times[name] = best
+    assert torch.isnan(audio).all()
+    assert times["nan"] <= 2 * times["numbers"], times
