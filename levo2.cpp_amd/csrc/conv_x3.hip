@@ -44,7 +44,8 @@
 // is summed again in plain F32, by the workgroup whose tile it is (f32_needed):
 // sums that are not finite where a finite product may overflow (its parts'
 // products overflow apart, or only the first does) or an operand is so small
-// that its first part may be zero. 20 to 40 times the tile's time.
+// that its first part may be zero, and tiles of operands so small that the parts
+// lose bits (bf16's smallest is 2^-133). 20 to 40 times the tile's time.
 #include "conv_x3.hpp"
 
 #include "snake_math.hpp"
@@ -298,25 +299,44 @@ __device__ __forceinline__ void join_sums(f32x16v & acc, const f32x16v & lo, flo
     }
 }
 
-// What a workgroup has seen; each wave's go into tile_state::seen.
-enum : uint32_t { kSumNotFinite = 1 };
+// What a workgroup has seen of its sums and operands; each wave's go into
+// tile_state::seen. "Ordinary" is large enough for a product with an ordinary
+// one of the other side to keep its bits.
+enum : uint32_t {
+    kSumNotFinite = 1,
+    kInputNonzero = 2, kInputOrdinary = 4,
+    kWeightNonzero = 8, kWeightOrdinary = 16,
+    kMidNonzero = 32, kMidOrdinary = 64,  // a residual unit's h
+    kWeight1Nonzero = 128, kWeight1Ordinary = 256,
+};
+constexpr float kOrdinaryInput = 0x1p-60f;
+constexpr float kOrdinaryWeight = 0x1p-40f;
 
 struct tile_state {
     uint32_t seen;
     // ranges over the tile (f32_needed)
-    uint32_t w, x_bound, x_infinite;
+    uint32_t w, x, x_bound, x_infinite;
     uint32_t mid, w1;
-    uint32_t pad[2];
+    uint32_t pad;
 };
 static_assert(sizeof(tile_state) == 32, "two items of LDS");
 
 __device__ __forceinline__ uint32_t seen_if(bool lane_has, uint32_t bit) { return __ballot(lane_has) != 0 ? bit : 0; }
 
-__device__ __forceinline__ bool worth_a_look(uint32_t seen) { return (seen & kSumNotFinite) != 0; }
+__device__ __forceinline__ bool worth_a_look(uint32_t seen) {
+    auto small = [&](uint32_t a, uint32_t a_ordinary, uint32_t b, uint32_t b_ordinary) {
+        return (seen & a) && (seen & b) && !((seen & a_ordinary) && (seen & b_ordinary));
+    };
+    return (seen & kSumNotFinite) || small(kInputNonzero, kInputOrdinary, kWeightNonzero, kWeightOrdinary) ||
+           small(kMidNonzero, kMidOrdinary, kWeight1Nonzero, kWeight1Ordinary);
+}
 
-// Whether sums of n products of values up to a and b may overflow.
-__device__ __forceinline__ bool out_of_split_range(float a, float b, float n) {
-    return a >= 0x1p126f || b >= 0x1p126f || a * b * n >= 0x1p126f;
+// Whether sums of n products of values up to a and b may overflow, or the values
+// or products be too small for their parts.
+__device__ __forceinline__ bool out_of_split_range(float a_bound, float a, float b, float n) {
+    const bool large = a_bound >= 0x1p126f || b >= 0x1p126f || a_bound * b * n >= 0x1p126f;
+    const bool small = a > 0.0f && b > 0.0f && (a < 0x1p-90f || b < 0x1p-90f || a * b < 0x1p-100f);
+    return large || small;
 }
 
 // The channel and phase of a row, its bias and output SnakeBeta, kept in LDS
@@ -396,6 +416,7 @@ __device__ __forceinline__ bool f32_needed(const x3_kernel_params & p, tile_stat
         }
     }
     atomicMax(&state->w, wr & ~kHasTiny);
+    atomicMax(&state->x, xr & ~kHasTiny);
     atomicMax(&state->x_bound, __builtin_bit_cast(uint32_t, bound));
     atomicOr(&state->x_infinite, (infinite ? 1u : 0u) | (xr & kHasTiny ? 2u : 0u) | (wr & kHasTiny ? 4u : 0u));
     __syncthreads();
@@ -403,8 +424,8 @@ __device__ __forceinline__ bool f32_needed(const x3_kernel_params & p, tile_stat
     // an infinity times a value whose first part may be zero (one of the weights
     // times a tiny input, or the other way)
     if ((state->seen & kSumNotFinite) && ((odd & 2) || (odd & 5) == 5)) return true;
-    return out_of_split_range(__builtin_bit_cast(float, state->x_bound), __builtin_bit_cast(float, state->w),
-                              static_cast<float>((ci1 - ci0) * KW));
+    return out_of_split_range(__builtin_bit_cast(float, state->x_bound), __builtin_bit_cast(float, state->x),
+                              __builtin_bit_cast(float, state->w), static_cast<float>((ci1 - ci0) * KW));
 }
 
 // The k = 1 half of a residual unit of 128 channels, in the k = 7 launch: a
@@ -515,14 +536,16 @@ __device__ __forceinline__ void unit_tail(const x3_kernel_params & p, u32x4 * ld
     };
     run_half(std::integral_constant<int, 0>{});
     run_half(std::integral_constant<int, 1>{});
-    seen |= seen_if(bad != 0.0f, kSumNotFinite);
+    seen |= seen_if(bad != 0.0f, kSumNotFinite) | seen_if(largest > 0.0f, kMidNonzero) |
+            seen_if(largest >= kOrdinaryInput, kMidOrdinary);
     if (lane == 0) atomicOr(&state->seen, seen);
     __syncthreads();
     if (!worth_a_look(state->seen)) return;
     atomicMax(&state->mid, __builtin_bit_cast(uint32_t, largest));
     if (tid < kUnit / 32 * (kUnit / kCI)) atomicMax(&state->w1, p.w1_range[tid] & ~kHasTiny);
     if (!f32_needed<7, kThreads>(p, state, 0, kUnit / 32, t0, 0, p.chunks) &&
-        !out_of_split_range(__builtin_bit_cast(float, state->mid), __builtin_bit_cast(float, state->w1), kUnit))
+        !out_of_split_range(__builtin_bit_cast(float, state->mid), __builtin_bit_cast(float, state->mid),
+                            __builtin_bit_cast(float, state->w1), kUnit))
         return;
     // plain F32, 32 columns of h at a time
     float * hs = reinterpret_cast<float *>(lds);
@@ -581,6 +604,20 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
     tile_state * state = reinterpret_cast<tile_state *>(lds + S::STATE);
     if (tid < static_cast<int>(sizeof(tile_state) / 4)) reinterpret_cast<uint32_t *>(state)[tid] = 0;
     uint32_t seen = 0;  // the wave's
+    {
+        uint32_t wr = 0, wr1 = 0;
+        const int g_begin = c_begin * S::CG;
+        const int n_ranges = S::WAVES * (c_end - c_begin) * S::CG;
+        for (int e = tid; e < n_ranges; e += S::THREADS) {
+            const int rt = row0 / 32 + e % S::WAVES;
+            if (rt * 32 < p.rows) wr = join_ranges(wr, p.w_range[rt * p.chunks * S::CG + g_begin + e / S::WAVES]);
+        }
+        if (FUSE && tid < kUnit / 32 * (kUnit / kCI)) wr1 = p.w1_range[tid];
+        auto at_least = [](uint32_t r, float v) { return (r & ~kHasTiny) >= __builtin_bit_cast(uint32_t, v); };
+        seen = seen_if(wr != 0, kWeightNonzero) | seen_if(at_least(wr, kOrdinaryWeight), kWeightOrdinary);
+        if (FUSE) seen |= seen_if(wr1 != 0, kWeight1Nonzero) | seen_if(at_least(wr1, kOrdinaryWeight), kWeight1Ordinary);
+    }
+    float largest = 0.0f;  // |input| staged by the thread
 
     // Staging: waves deal the columns, channel halves and groups of a chunk
     // among them, in pairs of channels; the eight channels of a column's item
@@ -636,6 +673,7 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
                 v[q] = exact ? snake(v[q], sp) : snake_fast(v[q], sp, slow);
             }
         }
+        largest = __builtin_fmaxf(__builtin_fmaxf(largest, __builtin_fabsf(v[0])), __builtin_fabsf(v[1]));
         uint32_t w[3];
         split2(v[0], v[1], w);
         u32x4 * item = lds + buf * S::BUF + u * S::GROUP + kg * S::W + col;
@@ -764,7 +802,8 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
             join_sums(acc[j], lo[j], tile_bad);
             if (32 * (j + 1) <= S::OUT || 32 * j + n < S::OUT) bad += tile_bad;
         }
-        seen = seen_if(bad != 0.0f, kSumNotFinite);
+        seen |= seen_if(bad != 0.0f, kSumNotFinite) | seen_if(largest > 0.0f, kInputNonzero) |
+                seen_if(largest >= kOrdinaryInput, kInputOrdinary);
     }
     if constexpr (FUSE) {
         unit_tail(p, lds, acc, state, seen, t0);

@@ -321,3 +321,28 @@ def test_nan_costs_no_more_than_numbers(hip, binding, dev, oracle):
         times[name] = best
     assert torch.isnan(audio).all()
     assert times["nan"] <= 2 * times["numbers"], times
+
+
+@pytest.mark.parametrize("xs,ws", [(-112, 0), (0, -112), (-70, -55), (-125, 0)])
+@pytest.mark.parametrize("kw,direct", [(7, True), (7, False), (2, True), (1, False)])
+def test_tiny_operands(hip, dev, oracle, kw, direct, xs, ws):
+    """Inputs or weights (or their products) that are all so small that the parts
+    would lose bits: as close to the exact sums as the F32 launch, in the 2-norm
+    relative to them (10 % and the smallest F32 steps allowed)."""
+    c, c_out, t, stride = (256, 256, 20000, 1) if kw != 2 else (512, 256, 3000, 4)
+    if kw == 2:
+        x, w, _, _, _ = _t_case(oracle, c, c_out, t, stride, 41)
+    else:
+        x, w, _, _, _, _ = _case(oracle, c, c_out, t, kw, 41)
+    x, w = x * np.float32(2.0 ** xs), w * np.float32(2.0 ** ws)
+    n = _direct_floats(c, c_out * stride, kw, t + 1) if direct else -1
+    if kw == 2:
+        got, plain = _run_t(hip, dev, x, w, None, 4, 2, ws_floats=n), _run_t(hip, dev, x, w, None, 4, 2, split=False)
+    else:
+        got, plain = (_run(hip, dev, x, w, None, kw // 2, 1, ws_floats=m) for m in (n, None))
+    rows = np.arange(0, c_out, 16)
+    exact = (_f64_transpose_rows(oracle, x, w, None, 4, 2, None, None, rows) if kw == 2 else
+             _f64_rows(oracle, x, w, None, kw // 2, 1, None, None, None, rows))
+    scale = 2.0 ** -(xs + ws)  # the sums of squares would underflow
+    err = lambda y: np.linalg.norm((y[rows].astype(np.float64) - exact) * scale)
+    assert err(got) <= 1.1 * err(plain) + c * kw * 2.0 ** -149 * scale * np.sqrt(exact.size)
