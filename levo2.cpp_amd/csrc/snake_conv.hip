@@ -1726,7 +1726,6 @@ int conv_transpose_entry(const float * x, int64_t x_stride, int64_t c_in, int64_
     p.splits = 1;
     if (ws != nullptr)
         LEVO_REQUIRE(aligned16(ws) && ws_floats >= 0, "conv_transpose1d: workspace must be 16-byte aligned");
-    if (thin_transpose(p)) return t_in < 8 ? launch_thin_transpose<8>(p, st, what) : launch_thin_transpose<16>(p, st, what);
     const int64_t wgs = ceil_div(t_in + 1, kNT) * ceil_div(c_out, kMT) * stride;
     const int64_t pitch = split_pitch(t_in + 1);
     int64_t splits = 1;
@@ -1736,13 +1735,16 @@ int conv_transpose_entry(const float * x, int64_t x_stride, int64_t c_in, int64_
         splits = pick_splits<2>(wgs, chunks, c_in, 1, snake, w_vec);
         while (splits > 1 && (chunks / splits < 2 || splits * stride * c_out * pitch > ws_floats)) --splits;
     }
-    if (const int rc = try_x3(p, 2, wgs, splits, ws, ws_floats, pack, st, what); rc != kNotX3) return rc;
     if (splits > 1) {
         const int64_t bytes = splits * stride * c_out * pitch * static_cast<int64_t>(sizeof(float));
         const int64_t elt = static_cast<int64_t>(sizeof(float));
         LEVO_REQUIRE(!ranges_overlap(ws, bytes, y, c_out * y_stride * elt) &&
                          !ranges_overlap(ws, bytes, x, c_in * x_stride * elt),
                      "conv_transpose1d: workspace overlaps a tensor");
+    }
+    if (thin_transpose(p)) return t_in < 8 ? launch_thin_transpose<8>(p, st, what) : launch_thin_transpose<16>(p, st, what);
+    if (const int rc = try_x3(p, 2, wgs, splits, ws, ws_floats, pack, st, what); rc != kNotX3) return rc;
+    if (splits > 1) {
         p.splits = static_cast<int32_t>(splits);
         p.part = ws;
         p.part_slice = c_out * pitch;

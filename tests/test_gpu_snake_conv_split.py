@@ -184,6 +184,18 @@ def test_rejects_bad_workspace(hip, dev, binding):
     assert hip.snake_conv1d_split_workspace_floats(3, 5) == 4 * 3 * 8
 
 
+def test_transpose_of_a_few_samples_rejects_bad_workspace(hip, dev, binding):
+    """The form that needs no partial sums refuses what the one with them does."""
+    import torch
+    c_in, c_out, t, s = 2048, 1024, 7, 10
+    x = torch.zeros((c_in, t), device=dev)
+    w = torch.zeros(s * c_out * c_in * 2, device=dev)
+    n = hip.snake_conv_transpose1d_split_workspace_floats(c_out, t, s)
+    ws = torch.zeros(n, device=dev)
+    with pytest.raises(binding.LevoHipError, match="overlaps"):
+        hip.snake_conv_transpose1d_split(x, c_in, t, w, c_out, s, workspace=ws, workspace_floats=n, padding=5, y=ws)
+
+
 # ---- transposed convolution (levo_hip_snake_conv_transpose1d_split) --------
 
 def _run_t(hip, dev, x, w, b, stride, pad, a=None, bl=None, param_type=0, split=True, ws_floats=-1):
