@@ -1445,6 +1445,44 @@ int64_t pick_splits(int64_t wgs, int64_t chunks, int64_t c_in, int64_t dil, bool
     return rounds_2 * 5 <= rounds_1 * 8 ? 2 : 1;                 // rounds_2 / 2 <= 0.8 rounds_1
 }
 
+// Whether a workspace meets anything the convolution reads or writes.
+bool meets_tensor(const conv_params & p, int kw, const float * ws, int64_t ws_floats) {
+    const int64_t elt = static_cast<int64_t>(sizeof(float));
+    const auto meets = [&](const void * t, int64_t bytes) {
+        return t != nullptr && ranges_overlap(ws, ws_floats * elt, t, bytes);
+    };
+    const int64_t param = p.param_f16 ? 2 : 4;
+    return meets(p.y, p.c_out * p.y_pitch * elt) || meets(p.x, p.c_in * p.x_pitch * elt) ||
+           meets(p.residual, p.c_out * p.r_pitch * elt) ||
+           meets(p.w, static_cast<int64_t>(p.o_stride) * p.c_out * p.c_in * kw * elt) || meets(p.bias, p.c_out * elt) ||
+           meets(p.alpha_log, p.c_in * param) || meets(p.beta_log, p.c_in * param) ||
+           meets(p.post_alpha_log, p.c_out * param) || meets(p.post_beta_log, p.c_out * param);
+}
+
+// The split count of p's F32 launch, from the one pick_splits wants: as many as
+// the workspace holds, of at least two K chunks each (`slice` floats of partial
+// sums a split). Partial sums that meet x, y or the residual are refused; splits
+// beyond kMaxSplits, which a caller with a workspace of ..._workspace_floats
+// never sees, are taken only where theirs meet nothing.
+int choose_splits(const conv_params & p, int kw, int64_t wanted, int64_t chunks, int64_t slice, const float * ws,
+                  int64_t ws_floats, const char * op, int64_t & splits) {
+    const auto fit = [&](int64_t n) {
+        while (n > 1 && (chunks / n < 2 || n * slice > ws_floats)) --n;
+        return n;
+    };
+    splits = fit(std::min<int64_t>(wanted, kMaxSplits));
+    if (splits > 1) {
+        const int64_t elt = static_cast<int64_t>(sizeof(float));
+        const int64_t bytes = splits * slice * elt;
+        LEVO_REQUIRE(!ranges_overlap(ws, bytes, p.y, p.c_out * p.y_pitch * elt) &&
+                         !ranges_overlap(ws, bytes, p.x, p.c_in * p.x_pitch * elt) &&
+                         (p.residual == nullptr || !ranges_overlap(ws, bytes, p.residual, p.c_out * p.r_pitch * elt)),
+                     "%s: workspace overlaps a tensor", op);
+    }
+    if (const int64_t more = fit(wanted); more > splits && !meets_tensor(p, kw, ws, more * slice)) splits = more;
+    return LEVO_HIP_OK;
+}
+
 // The bf16-split form of p (kernel kw, p.o_stride phases) where it takes the
 // convolution: its packed weights at the front of `pack` (or of the
 // workspace), its partial sums in the rest of it. Returns kNotX3
@@ -1479,12 +1517,8 @@ int try_x3(const conv_params & p, int kw, int64_t wgs, int64_t splits, float * w
         return launch_x3(c, kw, pack.p, pack.p + floats, part, st, what);
     }
     if (ws == nullptr || ws_floats < floats || x3_us(c, kw, ws_floats - floats) >= f32_us) return kNotX3;
-    // a workspace that meets a tensor is the F32 path's to judge
-    const int64_t elt = static_cast<int64_t>(sizeof(float));
-    if (ranges_overlap(ws, ws_floats * elt, p.y, p.c_out * p.y_pitch * elt) ||
-        ranges_overlap(ws, ws_floats * elt, p.x, p.c_in * p.x_pitch * elt) ||
-        (p.residual != nullptr && ranges_overlap(ws, ws_floats * elt, p.residual, p.c_out * p.r_pitch * elt)))
-        return kNotX3;
+    // the F32 launch may leave alone what a workspace shares with a tensor
+    if (meets_tensor(p, kw, ws, ws_floats)) return kNotX3;
     return launch_x3(c, kw, ws, ws + floats, ws_floats - floats, st, what);
 }
 
@@ -1566,19 +1600,16 @@ int conv1d_entry(const float * x, int64_t x_stride, int64_t c_in, int64_t t_in, 
             case 5: splits = pick_splits<5>(tiles, chunks, c_in, dilation, snake, w_vec); break;
             default: splits = pick_splits<7>(tiles, chunks, c_in, dilation, snake, w_vec); break;
         }
-        while (splits > 1 && (chunks / splits < 2 || splits * c_out * pitch > ws_floats)) --splits;
+        if (const int rc = choose_splits(p, static_cast<int>(kernel), splits, chunks, c_out * pitch, ws, ws_floats,
+                                         "snake_conv1d", splits);
+            rc != LEVO_HIP_OK)
+            return rc;
     }
     if (c_out > 4) {
         const int rc = try_x3(p, static_cast<int>(kernel), tiles, splits, ws, ws_floats, pack, st, what);
         if (rc != kNotX3) return rc;
     }
     if (splits > 1) {
-        const int64_t bytes = splits * c_out * pitch * static_cast<int64_t>(sizeof(float));
-        const int64_t elt = static_cast<int64_t>(sizeof(float));
-        LEVO_REQUIRE(!ranges_overlap(ws, bytes, y, c_out * y_stride * elt) &&
-                         !ranges_overlap(ws, bytes, x, c_in * x_stride * elt) &&
-                         (residual == nullptr || !ranges_overlap(ws, bytes, residual, c_out * residual_stride * elt)),
-                     "snake_conv1d: workspace overlaps a tensor");
         p.splits = static_cast<int32_t>(splits);
         p.part = ws;
         p.part_slice = c_out * pitch;
@@ -1733,14 +1764,9 @@ int conv_transpose_entry(const float * x, int64_t x_stride, int64_t c_in, int64_
         const int64_t chunks = ceil_div(c_in, conv_chunk<2>::CI);
         const bool w_vec = aligned16(packed_weight) && (c_in * 2) % 4 == 0 && (c_out * c_in * 2) % 4 == 0;
         splits = pick_splits<2>(wgs, chunks, c_in, 1, snake, w_vec);
-        while (splits > 1 && (chunks / splits < 2 || splits * stride * c_out * pitch > ws_floats)) --splits;
-    }
-    if (splits > 1) {
-        const int64_t bytes = splits * stride * c_out * pitch * static_cast<int64_t>(sizeof(float));
-        const int64_t elt = static_cast<int64_t>(sizeof(float));
-        LEVO_REQUIRE(!ranges_overlap(ws, bytes, y, c_out * y_stride * elt) &&
-                         !ranges_overlap(ws, bytes, x, c_in * x_stride * elt),
-                     "conv_transpose1d: workspace overlaps a tensor");
+        if (const int rc = choose_splits(p, 2, splits, chunks, stride * c_out * pitch, ws, ws_floats, "conv_transpose1d", splits);
+            rc != LEVO_HIP_OK)
+            return rc;
     }
     if (thin_transpose(p)) return t_in < 8 ? launch_thin_transpose<8>(p, st, what) : launch_thin_transpose<16>(p, st, what);
     if (const int rc = try_x3(p, 2, wgs, splits, ws, ws_floats, pack, st, what); rc != kNotX3) return rc;

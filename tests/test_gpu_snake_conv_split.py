@@ -184,6 +184,34 @@ def test_rejects_bad_workspace(hip, dev, binding):
     assert hip.snake_conv1d_split_workspace_floats(3, 5) == 4 * 3 * 8
 
 
+@pytest.mark.parametrize("where", ["x", "weight"])
+def test_workspace_that_meets_a_tensor_past_the_splits(hip, dev, oracle, where):
+    """Splits beyond the four that the workspace query counts, and the split
+    weights of the bf16 form, leave alone what the workspace shares with a tensor
+    where four partial sums (or none) do not reach: the call stays accepted, with
+    the bits of the same call in a workspace that ends there."""
+    import torch
+    c, t, kw = (1024, 70, 1) if where == "x" else (256, 30000, 7)
+    x, w, b, a, bl, _ = _case(oracle, c, c, t, kw, 61)
+    n = 4 * c * ((t + 3) // 4 * 4) if where == "x" else 0
+    want = _run(hip, dev, x, w, b, kw // 2, 1, a, bl, ws_floats=n or None)
+    big = torch.zeros(40 * c * 72 if where == "x" else 2 * c * t, device=dev)
+    xd, wd = to_dev(x, dev), to_dev(w, dev)
+    moved = xd if where == "x" else wd
+    inside = big[n:n + moved.numel()].view(moved.shape)
+    inside.copy_(moved)
+    if where == "x":
+        xd = inside
+    else:
+        wd = inside
+    y = torch.empty((c, t), device=dev)
+    hip.snake_conv1d_split(xd, c, t, wd, c, kw, workspace=big, workspace_floats=big.numel(), alpha_log=to_dev(a, dev),
+                           beta_log=to_dev(bl, dev), bias=to_dev(b, dev), padding=kw // 2, y=y)
+    torch.cuda.synchronize()
+    assert np.array_equal(from_dev(y).view(np.uint32), want.view(np.uint32))
+    assert torch.equal(inside, moved)
+
+
 def test_transpose_of_a_few_samples_rejects_bad_workspace(hip, dev, binding):
     """The form that needs no partial sums refuses what the one with them does."""
     import torch
