@@ -1002,9 +1002,11 @@ x3_layout layout_of(const x3_conv & c, int kw) {
 // A residual unit's k = 1 weights in fragment order.
 constexpr int64_t kUnitFragBytes = kUnit / 32 * (kUnit / kCI) * 3072;
 
-// Fewer multiply-adds than this (16 us at the F32 launches' 100 TFLOP/s) are not
-// worth the pack launch of about 5 us.
-constexpr int64_t kMinMacs = 800'000'000;
+// Fewer multiply-adds than this (8 us at the F32 launches' 100 TFLOP/s) are not
+// worth the pack launch of about 5 us; nor are those of a residual unit, one
+// launch in F32 too, below twice as many.
+constexpr int64_t kMinMacs = 400'000'000;
+constexpr int64_t kMinUnitMacs = 800'000'000;
 
 // Microseconds of a launch with `splits` splits: rounds of one workgroup a CU
 // at 0.075 us per K value (measured with every CU busy: 512 channels x 60000,
@@ -1100,16 +1102,25 @@ int64_t x3_pack_bytes(const x3_conv & c, int kw) {
     if (static_cast<int64_t>(c.c_out) * c.stride <= 128) return -1;
     if (c.c_out > (1 << 16) || c.c_in > (1 << 16) || c.cols >= (int64_t{1} << 28)) return -1;
     const double macs = static_cast<double>(c.c_out) * c.stride * c.c_in * kw * static_cast<double>(c.cols);
-    if (macs < kMinMacs / 2) return -1;
+    if (macs < kMinMacs) return -1;
     return layout_of(c, kw).bytes();
 }
 
+// Fitted like the F32 launches' estimate (snake_conv.hip): rounds of one
+// workgroup a CU on the fullest XCD, the partial sums' way through memory, the
+// pack launch; split weights that the 256 MB last-level cache cannot hold with
+// what they are made from come from memory again.
 double x3_us(const x3_conv & c, int kw, int64_t part_floats) {
     const x3_layout l = layout_of(c, kw);
     const int64_t tiles = ceil_div(c.cols, kw == 2 ? kNT - 1 : kNT) * ceil_div(l.rows, 256);
     double us;
-    pick_splits(c, l, tiles, l.groups * kCI * kw, part_floats, us);
-    return us + 5.0 + static_cast<double>(l.frag_bytes) / 2.6e6;  // the pack launch
+    const int splits = pick_splits(c, l, tiles, l.groups * kCI * kw, part_floats, us);
+    const double k_us = kw == 1 ? 0.087 : kw == 2 ? 0.067 : kw == 3 ? 0.061 : 0.050;
+    const double share = static_cast<double>(ceil_div(l.chunks, splits) * (l.groups / l.chunks) * kCI * kw);
+    const double rounds = static_cast<double>(ceil_div(ceil_div(tiles, 8) * splits, 32));
+    const double part_mb = splits > 1 ? 4.0e-6 * static_cast<double>(splits * l.rows * ((c.cols + 3) / 4 * 4)) : 0.0;
+    const double frag_mb = 1.0e-6 * static_cast<double>(l.frag_bytes);
+    return (kw == 2 ? 6.0 : 3.0) + rounds * (k_us * share + 11.0) + 0.4 * part_mb + (frag_mb < 128.0 ? 0.43 : 0.6) * frag_mb;
 }
 
 int launch_x3(const x3_conv & c, int kw, void * pack, float * part, int64_t part_floats, hipStream_t st,
@@ -1127,7 +1138,7 @@ int launch_x3(const x3_conv & c, int kw, void * pack, float * part, int64_t part
 int64_t x3_unit_pack_bytes(const x3_conv & c) {
     if (c.c_in != kUnit || c.c_out != kUnit || c.stride != 1 || !c.snake || !c.post_alpha_log || c.residual ||
         static_cast<int64_t>(c.dil) * 6 > kMaxHalo || c.cols >= (int64_t{1} << 28) ||
-        c.cols * kUnit * kUnit * 8 < kMinMacs)
+        c.cols * kUnit * kUnit * 8 < kMinUnitMacs)
         return -1;
     return layout_of(c, 7).bytes() + kUnitFragBytes + round16(4 * (kUnit / 32) * (kUnit / kCI));
 }

@@ -1483,34 +1483,48 @@ int choose_splits(const conv_params & p, int kw, int64_t wanted, int64_t chunks,
     return LEVO_HIP_OK;
 }
 
+// Microseconds of p's F32 launch in `splits` splits (and of its combine), where
+// that can be less than the bf16 form's: in grids that leave compute units
+// idle. Fitted to 1400 launches of 0.4 to 16 G multiply-adds (64 to 2048
+// channels, 1 to 60000 samples, 1 to 32 splits), nine in ten within 5 %: a share
+// of K at a rate that a second workgroup on the CU slows down, by the fullest
+// XCD (32 CUs; a tile's phases and splits are one XCD's), 0.46 us per MB of
+// partial sums, and more where the weights cannot be loaded 16 bytes at a time.
+double f32_launch_us(const conv_params & p, int kw, int64_t splits) {
+    const int64_t tiles = ceil_div(p.t_out, kNT) * ceil_div(p.c_out, kMT);
+    if (tiles * p.o_stride >= std::max(1, device_cu_count())) return 1e30;
+    const int64_t ci = kw == 1 ? conv_chunk<1>::CI : kw == 2 ? conv_chunk<2>::CI : conv_chunk<7>::CI;
+    const double share = static_cast<double>(ceil_div(ceil_div(p.c_in, ci), splits) * ci * kw);
+    const int64_t per_xcd = ceil_div(tiles, 8) * p.o_stride * splits;
+    const bool alone = per_xcd <= 32;
+    double k_us, fixed;
+    switch (kw) {
+        case 1: k_us = alone ? 0.194 : 0.245, fixed = 12.0; break;
+        case 2: k_us = alone ? 0.092 : 0.173, fixed = 20.0; break;
+        case 3: k_us = alone ? 0.163 : 0.214, fixed = 13.0; break;
+        default: k_us = alone ? 0.088 : 0.143, fixed = 12.0; break;
+    }
+    if (!aligned16(p.w) || static_cast<int64_t>(p.c_in) * kw % 4 != 0)
+        k_us *= kw == 2 || kw == 7 ? (alone ? 1.6 : 1.45) : (alone ? 1.15 : 1.1);  // k 2 and 7 lose the interleaved kernel
+    const double rounds = alone ? 1.0 : static_cast<double>(ceil_div(per_xcd, 64));
+    const double part_mb = splits > 1 ? 4.0e-6 * static_cast<double>(splits * p.o_stride * p.c_out * ((p.t_out + 3) / 4 * 4)) : 0.0;
+    return fixed + rounds * k_us * share + 0.46 * part_mb;
+}
+
 // The bf16-split form of p (kernel kw, p.o_stride phases) where it takes the
 // convolution: its packed weights at the front of `pack` (or of the
 // workspace), its partial sums in the rest of it. Returns kNotX3
-// with nothing launched where it does not.
+// with nothing launched where it does not. Of 1690 shapes timed in either form, 12
+// take the slower one by more than 2 % (the worst by 15 %, 253 for 219 us).
 constexpr int kNotX3 = 1;
 
-// Microseconds of the F32 launch with `wgs` workgroups in `splits` splits,
-// where that can be less than the bf16-split one's: grids that leave compute
-// units idle, whose bf16 form is short of partial-sum space (its packed weights
-// take part of the same workspace). Measured per K value of a workgroup's share:
-// k = 7 0.09 us alone on a CU, 0.15 us with a second one (1024 channels x 800
-// and x 2520, 512 x 1600 and x 2520), k = 2 0.16 and 0.25 us; k = 1 and 3 stayed
-// slower than the bf16 form at every length measured (800 to 240000 samples).
-double f32_launch_us(int kw, int64_t wgs, int64_t splits, int64_t c_in) {
-    const int64_t cus = std::max(1, device_cu_count());
-    if (kw == 1 || kw == 3 || wgs >= cus) return 1e30;
-    const double share = static_cast<double>(c_in * kw) / static_cast<double>(splits);
-    const bool alone = wgs * splits <= cus;
-    return share * (kw == 7 ? (alone ? 0.09 : 0.15) : (alone ? 0.16 : 0.25)) + 6.0;
-}
-
-int try_x3(const conv_params & p, int kw, int64_t wgs, int64_t splits, float * ws, int64_t ws_floats,
+int try_x3(const conv_params & p, int kw, int64_t splits, float * ws, int64_t ws_floats,
            const scratch_span & pack, hipStream_t st, const char * what) {
     const x3_conv c = x3_of(p);
     const int64_t bytes = x3_pack_bytes(c, kw);
     if (bytes < 0) return kNotX3;
     const int64_t floats = ceil_div(bytes, 16) * 4;
-    const double f32_us = f32_launch_us(kw, wgs, splits, p.c_in);
+    const double f32_us = f32_launch_us(p, kw, splits);
     if (pack.p != nullptr && pack.floats >= floats) {
         const int64_t part = pack.floats - floats;
         if (x3_us(c, kw, part) >= f32_us) return kNotX3;
@@ -1606,7 +1620,7 @@ int conv1d_entry(const float * x, int64_t x_stride, int64_t c_in, int64_t t_in, 
             return rc;
     }
     if (c_out > 4) {
-        const int rc = try_x3(p, static_cast<int>(kernel), tiles, splits, ws, ws_floats, pack, st, what);
+        const int rc = try_x3(p, static_cast<int>(kernel), splits, ws, ws_floats, pack, st, what);
         if (rc != kNotX3) return rc;
     }
     if (splits > 1) {
@@ -1769,7 +1783,7 @@ int conv_transpose_entry(const float * x, int64_t x_stride, int64_t c_in, int64_
             return rc;
     }
     if (thin_transpose(p)) return t_in < 8 ? launch_thin_transpose<8>(p, st, what) : launch_thin_transpose<16>(p, st, what);
-    if (const int rc = try_x3(p, 2, wgs, splits, ws, ws_floats, pack, st, what); rc != kNotX3) return rc;
+    if (const int rc = try_x3(p, 2, splits, ws, ws_floats, pack, st, what); rc != kNotX3) return rc;
     if (splits > 1) {
         p.splits = static_cast<int32_t>(splits);
         p.part = ws;

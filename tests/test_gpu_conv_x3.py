@@ -346,3 +346,46 @@ def test_tiny_operands(hip, dev, oracle, kw, direct, xs, ws):
     scale = 2.0 ** -(xs + ws)  # the sums of squares would underflow
     err = lambda y: np.linalg.norm((y[rows].astype(np.float64) - exact) * scale)
     assert err(got) <= 1.1 * err(plain) + c * kw * 2.0 ** -149 * scale * np.sqrt(exact.size)
+
+
+@pytest.mark.parametrize("c_in,c_out,kw,dil,t,stride,big", [
+    (1024, 1024, 1, 1, 573, 0, False), (2048, 512, 1, 1, 1146, 0, False), (512, 512, 3, 1, 763, 0, False),
+    (256, 256, 7, 9, 3120, 0, True), (256, 256, 7, 1, 2616, 0, True), (2048, 1024, 2, 1, 50, 10, True),
+    (2048, 1024, 2, 1, 100, 10, True), (512, 512, 7, 3, 15121, 0, True), (1024, 1024, 7, 9, 2520, 0, True),
+    (2048, 1024, 2, 1, 1000, 10, True)])
+def test_route_is_the_faster_one(hip, dev, oracle, c_in, c_out, kw, dil, t, stride, big):
+    """The form that the estimates choose, in the queried workspace or a large
+    one, against the F32 launch with its four splits, which the same call takes
+    where the workspace meets a tensor past the partial sums (here the bias):
+    no slower, within 10 % for the clock and what the estimates cannot see."""
+    import torch
+    rows = c_out * max(stride, 1)
+    cols = t + 1 if stride else t
+    n = 4 * rows * ((cols + 3) // 4 * 4)
+    n = n + 100_000_000 if big else n
+    ws = torch.zeros(n + c_out, device=dev)
+    g = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn(c_in, t, device=dev, generator=g)
+    w = torch.randn(rows * c_in * kw, device=dev, generator=g) * 0.02
+    params = dict(alpha_log=torch.zeros(c_in, device=dev), beta_log=torch.zeros(c_in, device=dev))
+    pad = (stride + 1) // 2 if stride else dil * (kw - 1) // 2
+    y = torch.empty((c_out, (t + 1) * stride - 2 * pad if stride else t), device=dev)
+
+    def call(floats):
+        kwargs = dict(workspace=ws, workspace_floats=floats, bias=ws[n:], padding=pad, y=y, **params)
+        if stride:
+            hip.snake_conv_transpose1d_split(x, c_in, t, w, c_out, stride, **kwargs)
+        else:
+            hip.snake_conv1d_split(x, c_in, t, w, c_out, kw, dilation=dil, **kwargs)
+
+    best = {n: 1e9, n + c_out: 1e9}
+    for _ in range(8):
+        for floats in best:
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(5):
+                call(floats)
+            b.record()
+            b.synchronize()
+            best[floats] = min(best[floats], a.elapsed_time(b) / 5)
+    assert best[n] <= 1.1 * best[n + c_out], best
