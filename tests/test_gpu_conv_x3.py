@@ -71,6 +71,21 @@ def test_falls_back(hip, dev, oracle):
         assert np.array_equal(got.view(np.uint32), plain.view(np.uint32))
 
 
+@pytest.mark.parametrize("c_in,kw", [(1, 3), (2, 1)])
+def test_sums_of_few_terms_stay_in_f32(hip, dev, c_in, kw):
+    """Below four terms the F32 launch is the closer one: its bits."""
+    import torch
+    c_out = 512
+    t = 420_000_000 // (c_out * c_in * kw)
+    g = torch.Generator(device=dev).manual_seed(4)
+    x, w = torch.randn(c_in, t, device=dev, generator=g), torch.randn(c_out, c_in, kw, device=dev, generator=g)
+    got, plain = torch.empty(c_out, t, device=dev), torch.empty(c_out, t, device=dev)
+    ws = torch.empty(4 * c_out * kw * 64, device=dev)  # the split weights and no partial sum
+    hip.snake_conv1d_split(x, c_in, t, w, c_out, kw, workspace=ws, workspace_floats=ws.numel(), padding=kw // 2, y=got)
+    hip.snake_conv1d(x, c_in, t, w, c_out, kw, padding=kw // 2, y=plain)
+    assert torch.equal(got, plain)
+
+
 def test_f16_params_large_arguments_in_place_residual(hip, dev, oracle):
     """|alpha x| beyond the reduced sine's 8192 in some channels; y written over
     the residual."""
