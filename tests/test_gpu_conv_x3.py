@@ -6,13 +6,16 @@ is large enough and the workspace holds the split weights.
 Bars: max |y - exact| / max(|exact|, 1) <= 1e-5 against the convolution of the
 oracle's SnakeBeta output in float64, the bar of the F32 launches, and in the
 2-norm no further from it than the F32 launch of the same data (the split
-operands are exact, the products left out are below 2^-25 of a product, and the
+operands are exact, the products left out are below 2^-24 of a product, and the
 sums round once per 16 terms where the F32 MFMA rounds once per 4). The route is
-checked too: another order of the sums gives other bits than the F32 launch.
+checked too: another order of the sums gives other bits than the F32 launch,
+whose grid is full where a test says that the epilogue is the direct one.
 Shapes: partial row tiles (129, 200, 257 output channels) and channel groups,
 column tiles of 128 (127 for the transposed form) with remainders, the widest
 halo (dilation 10) and the first beyond it (11, which keeps the F32 launch),
-strides, F16 parameters, arguments beyond the reduced sine, y over the residual.
+strides, F16 parameters, arguments beyond the reduced sine, y over the residual,
+each with partial sums (the queried workspace) and in one split (`direct`);
+whole decodes of windows that take every form; special, tiny and huge values.
 """
 from __future__ import annotations
 
@@ -25,6 +28,12 @@ from test_gpu_vae_decoder import device_weights
 from vae_chain import Weights, decode_f64, scaled_err
 
 pytestmark = pytest.mark.gpu
+
+
+def _direct_floats(c_in, rows, kw, cols):
+    """Workspace for the split weights and less than two partial sums: one split, the direct epilogue."""
+    pack = -(-rows // 32) * 32 * -(-c_in // 32) * 32 * kw * 3 // 2
+    return pack + pack // 64 + 8 * (c_in + rows) + 64 + rows * cols
 
 
 def _compare(got, plain, exact, rows):
@@ -86,15 +95,17 @@ def test_sums_of_few_terms_stay_in_f32(hip, dev, c_in, kw):
     assert torch.equal(got, plain)
 
 
-def test_f16_params_large_arguments_in_place_residual(hip, dev, oracle):
+@pytest.mark.parametrize("t,direct", [(12345, False), (16741, True)])
+def test_f16_params_large_arguments_in_place_residual(hip, dev, oracle, t, direct):
     """|alpha x| beyond the reduced sine's 8192 in some channels; y written over
     the residual."""
-    c, t = 256, 12345
+    c = 256
     x, w, b, a, bl, r = _case(oracle, c, c, t, 7, 9, True)
     x[::5, ::7] *= np.float32(3e4)
     a16, b16 = oracle.f32_to_f16(a), oracle.f32_to_f16(bl)
     a32, b32 = oracle.f16_to_f32(a16), oracle.f16_to_f32(b16)
-    got = _run(hip, dev, x, w, b, 9, 3, a16, b16, r, param_type=1, in_place=True)
+    got = _run(hip, dev, x, w, b, 9, 3, a16, b16, r, param_type=1, in_place=True,
+               ws_floats=_direct_floats(c, c, 7, t) if direct else -1)
     plain = _run(hip, dev, x, w, b, 9, 3, a16, b16, r, param_type=1, ws_floats=None)
     rows = np.arange(0, c, 16)
     exact = _f64_rows(oracle, x, w, b, 9, 3, a32, b32, r, rows)
@@ -103,37 +114,47 @@ def test_f16_params_large_arguments_in_place_residual(hip, dev, oracle):
     assert np.linalg.norm(got[rows] - exact) <= np.linalg.norm(plain[rows] - exact)
 
 
-def test_strides(hip, dev, oracle):
+@pytest.mark.parametrize("t,direct", [(12001, False), (16641, True)])
+def test_strides(hip, dev, oracle, t, direct):
     """x, residual and y rows further apart than their samples, none aligned."""
     import torch
-    c, t, kw = 256, 12001, 7
+    c, kw = 256, 7
     x, w, b, a, bl, r = _case(oracle, c, c, t, kw, 11, True)
     xd = torch.full((c, t + 5), float("nan"), device=dev)
     rd = torch.full((c, t + 3), float("nan"), device=dev)
     yd = torch.full((c, t + 9), 7.0, device=dev)
     xd[:, :t], rd[:, :t] = to_dev(x, dev), to_dev(r, dev)
-    n = hip.snake_conv1d_split_workspace_floats(c, t)
+    n = _direct_floats(c, c, kw, t) if direct else hip.snake_conv1d_split_workspace_floats(c, t)
     ws = torch.full((n,), float("nan"), device=dev)
     hip.snake_conv1d_split(xd, c, t, to_dev(w, dev), c, kw, workspace=ws, workspace_floats=n, x_stride=t + 5,
                            alpha_log=to_dev(a, dev), beta_log=to_dev(bl, dev), bias=to_dev(b, dev), padding=3,
                            residual=rd, residual_stride=t + 3, y=yd, y_stride=t + 9)
     torch.cuda.synchronize()
     got = from_dev(yd)
-    assert np.array_equal(got[:, :t], _run(hip, dev, x, w, b, 3, 1, a, bl, r))
+    assert np.array_equal(got[:, :t], _run(hip, dev, x, w, b, 3, 1, a, bl, r, ws_floats=n))
+    assert not np.array_equal(got[:, :t], _run(hip, dev, x, w, b, 3, 1, a, bl, r, ws_floats=None))
     assert np.all(got[:, t:] == 7.0)
 
 
-@pytest.mark.parametrize("kw,where", [(7, "x"), (1, "x"), (7, "w"), (2, "x"), (2, "w")])
-def test_values_that_cannot_be_split(hip, dev, oracle, kw, where):
+@pytest.mark.parametrize("kw,where,direct,snake", [
+    (7, "x", False, False), (1, "x", False, False), (7, "w", False, False), (2, "x", False, False), (2, "w", False, False),
+    (7, "x", True, False), (7, "w", True, True), (2, "x", True, True), (2, "w", True, False), (7, "x", True, True),
+    (7, "x", False, True), (1, "w", True, True), (7, "w not finite", True, True), (2, "w not finite", False, False),
+    (7, "w not finite", False, False), (1, "w not finite", True, False)])
+def test_values_that_cannot_be_split(hip, dev, oracle, kw, where, direct, snake):
     """Infinities, NaN and a finite value that rounds to a bf16 infinity, in the
-    input and in the weights: the same infinities and NaN as the F32 launch, the
-    other outputs within the F32 bar."""
-    c, t = (256, 20000) if kw != 2 else (512, 3000)
-    big = (np.inf, -np.inf, np.nan, np.float32(3.4e38))
+    input and in the weights, with SnakeBeta (which makes NaN of an infinity) and
+    without: the same infinities and NaN as the F32 launch, the other outputs
+    within the F32 bar."""
+    c, t = (256, 20000) if kw != 2 else (512, 4300)
+    big = (np.inf, -np.inf, np.nan, np.float32(3.4e38))[:3 if where == "w not finite" else 4]
     if kw == 2:
-        x, w, b, _, _ = _t_case(oracle, c, 256, t, 4, 21)
+        x, w, b, a, bl = _t_case(oracle, c, 256, t, 4, 21)
     else:
-        x, w, b, _, _, _ = _case(oracle, c, c, t, kw, 21)
+        x, w, b, a, bl, _ = _case(oracle, c, c, t, kw, 21)
+    if not snake:
+        a = bl = None
+    n = _direct_floats(c, c if kw != 2 else 1024, kw, t + 1) if direct else -1
     for i, v in enumerate(big):
         if where == "x":
             x[3 + 17 * i, 100 + 700 * i] = v
@@ -142,16 +163,13 @@ def test_values_that_cannot_be_split(hip, dev, oracle, kw, where):
         else:
             w[5 + 40 * i, 3 + 17 * i, i % kw] = v
     if kw == 2:
-        got, plain = (_run_t(hip, dev, x, w, b, 4, 2, split=s) for s in (True, False))
+        got = _run_t(hip, dev, x, w, b, 4, 2, a, bl, ws_floats=n)
+        plain = _run_t(hip, dev, x, w, b, 4, 2, a, bl, split=False)
     else:
-        got, plain = (_run(hip, dev, x, w, b, kw // 2, 1, ws_floats=n) for n in (-1, None))
+        got, plain = (_run(hip, dev, x, w, b, kw // 2, 1, a, bl, ws_floats=m) for m in (n, None))
+    # the bf16 route: other bits where all is finite (3.4e38 in the weights has every tile summed in F32)
+    assert where == "w" or not np.array_equal(got[:, 4000:].view(np.uint32), plain[:, 4000:].view(np.uint32))
     _same_or_close(got, plain)
-
-
-def _direct_floats(c_in, rows, kw, cols):
-    """Workspace for the split weights and less than two partial sums: one split, the direct epilogue."""
-    pack = -(-rows // 32) * 32 * -(-c_in // 32) * 32 * kw * 3 // 2
-    return pack + pack // 64 + 8 * (c_in + rows) + 64 + rows * cols
 
 
 def _same_or_close(got, plain):
@@ -177,7 +195,7 @@ def test_products_that_overflow(hip, dev, oracle, kw, direct):
     parts of the split operands overflow with either sign, and by so little that
     only the product of their first parts does): the infinities, NaN and finite
     values of the F32 launch, in one split and in several."""
-    c, c_out, t, stride = (256, 256, 20000, 1) if kw != 2 else (512, 256, 3000, 4)
+    c, c_out, t, stride = (256, 256, 20000, 1) if kw != 2 else (512, 256, 4300, 4)
     if kw == 2:
         x, w, b, _, _ = _t_case(oracle, c, c_out, t, stride, 31)
     else:
@@ -208,14 +226,102 @@ def _decode(hip, dev, dw, latent, frames, stage5):
     return from_dev(out if stage5 else audio)
 
 
-@pytest.mark.parametrize("frames", [7, 17])
+def _f64_decode(w, latent, dev):
+    """vae_chain's decode_f64 with torch on the GPU: one product per tap."""
+    import torch
+    put = lambda a: to_dev(a, dev).double()
+
+    def snake(x, ab):
+        return x + torch.sin(torch.exp(put(ab[0]))[:, None] * x) ** 2 / (torch.exp(put(ab[1])) + 1e-9)[:, None]
+
+    def conv(x, wt, bias, dil):
+        k, t = wt.shape[2], x.shape[1]
+        xp = torch.nn.functional.pad(x, (dil * (k - 1) // 2, dil * (k - 1) // 2))
+        y = sum(put(wt[:, :, j]) @ xp[:, j * dil:j * dil + t].contiguous() for j in range(k))
+        return y if bias is None else y + put(bias)[:, None]
+
+    def upsample(x, wt, bias, stride):
+        t = x.shape[1]
+        full = x.new_zeros(wt.shape[1], t + 1, stride)
+        for r in range(stride):
+            full[:, :t, r] += put(wt[:, :, r].T) @ x
+            full[:, 1:, r] += put(wt[:, :, r + stride].T) @ x
+        pad = (stride + 1) // 2
+        return full.reshape(wt.shape[1], -1)[:, pad:(t + 1) * stride - pad] + put(bias)[:, None]
+
+    h = conv(put(latent), *w.input, 1)
+    for stage, stride in zip(w.stages, (10, 6, 4, 4, 2)):
+        h = upsample(snake(h, stage["act"]), *stage["up"], stride)
+        for unit, dil in zip(stage["res"], (1, 3, 9)):
+            h = h + conv(snake(conv(snake(h, unit["pre"]), *unit["conv0"], dil), unit["post"]), *unit["conv1"], 1)
+    return conv(snake(h, w.out_act), w.out_w, None, 1)
+
+
+@pytest.mark.parametrize("frames", [7, 17, 24, 64, 110, 252, 1000])
 def test_decoder(hip, binding, dev, oracle, frames):
-    """One-launch residual units of stages 4 and 5 (7 frames), also stage 1 - 3
-    convolutions and upsamplers (17): within the decoder's bar against float64."""
+    """Windows of every route (test_decoder_takes_every_form) against float64:
+    the decoder's bar at the signal's scale, and in the 2-norm 1.2e-6, which the
+    F32 launches keep to."""
+    import torch
     w = Weights(binding, 50 + frames)
     latent = oracle.gaussian(64 * frames, frames).reshape(64, frames)
     dw, keep = device_weights(hip, binding, dev, w)
-    assert scaled_err(_decode(hip, dev, dw, latent, frames, False), decode_f64(w, latent)) <= 1e-5
+    got = _decode(hip, dev, dw, latent, frames, False).astype(np.float64)
+    exact = _f64_decode(w, latent, dev).cpu().numpy()
+    if frames == 7:
+        assert scaled_err(exact, decode_f64(w, latent)) <= 1e-12
+    assert scaled_err(got, exact) <= 1e-5
+    assert np.linalg.norm(got - exact) <= 1.2e-6 * np.linalg.norm(exact)
+
+
+def test_decoder_takes_every_form(hip, binding, dev, oracle):
+    """The launches of the windows above: k = 7 and k = 1 convolutions of stages 1
+    to 3 and the upsamplers with partial sums and without, the units of stages 4
+    and 5, both narrow outputs, the thin upsampler."""
+    import re
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    w = Weights(binding, 51)
+    dw, keep = device_weights(hip, binding, dev, w)
+    forms = {}
+    for frames in (7, 24, 110, 252, 1000):
+        latent = oracle.gaussian(64 * frames, frames).reshape(64, frames)
+        _decode(hip, dev, dw, latent, frames, False)
+        with profile(activities=[ProfilerActivity.CUDA]) as prof:
+            _decode(hip, dev, dw, latent, frames, False)
+        events = sorted((e for e in prof.events() if "levo_hip::" in e.name), key=lambda e: e.time_range.start)
+        if not events:
+            pytest.skip("no kernel events from the profiler")
+        names = [re.sub(r"\(anonymous namespace\)::|levo_hip::|void |\(.*", "", e.name.replace("(anonymous namespace)::", ""))
+                 for e in events]
+        forms[frames] = {n + (" + combine" if i + 1 < len(names) and "combine" in names[i + 1] else "")
+                         for i, n in enumerate(names)}
+    k7, k1, up, unit = ("x3_conv_kernel<%s>" % a for a in ("7, true, false", "1, false, false", "2, true, false",
+                                                           "7, true, true"))
+    assert {"thin_transpose_kernel<8>", k7 + " + combine", up + " + combine", unit,
+            "snake_conv_narrow_kernel<7, 2, 1>"} <= forms[7]
+    assert {k7 + " + combine", up + " + combine"} <= forms[24]
+    assert {k7, k7 + " + combine", k1, k1 + " + combine", up, up + " + combine"} <= forms[110]
+    assert {k7, k1, up, unit, "snake_conv_narrow_kernel<7, 2, 4>"} <= forms[252]
+    assert {k7, k1, up, unit} <= forms[1000] and not any("scatter" in n for n in forms[1000])
+
+
+@pytest.mark.parametrize("frames", [24, 110])
+def test_stage_with_large_inner_values(hip, binding, dev, oracle, frames):
+    """Stage 3 with values between its convolutions whose sine arguments pass the
+    reduced form's range: the SnakeBeta that the k = 7 convolution stores is
+    evaluated anew there, in the combine (24 frames) and in the direct epilogue
+    (110). Against the public F32 calls from the decode's own stage 2 output."""
+    w = Weights(binding, 90)
+    for unit in w.stages[2]["res"]:
+        unit["conv0"][1][::9] = np.float32(3e4)
+        unit["conv1"][0][:, ::9] *= np.float32(1e-4)
+    latent = oracle.gaussian(64 * frames, 13).reshape(64, frames)
+    dw, keep = device_weights(hip, binding, dev, w)
+    got, plain = _stage(hip, binding, dev, w, dw, latent, frames, 2)
+    assert np.all(np.isfinite(plain))
+    # an inner value of 3e4 is known to 4e-3, its sine's square to 8e-3, and counts 1e-4 times: below the sums' rounding
+    assert f32_err(got, plain) <= 2e-5
 
 
 def test_unit_with_a_weight_that_cannot_be_split(hip, binding, dev, oracle):
@@ -255,25 +361,29 @@ def test_unit_with_products_that_overflow(hip, binding, dev, oracle):
         assert f32_err(after[others], before[others]) <= 1e-5
 
 
-def _last_stage(hip, binding, dev, w, dw, latent, frames):
-    """Stage 5 as the decode computes it (one-launch bf16 units), and from the
-    decode's stage 4 output by the public upsampler and residual units (F32)."""
+def _stage(hip, binding, dev, w, dw, latent, frames, s):
+    """Stage s (from 0) as the decode computes it, and from the decode's output of
+    the stage before by the public upsampler and residual units (F32)."""
     import torch
     nbytes = hip.vae_decode_workspace_bytes(frames)
     ws = torch.full((nbytes // 4,), float("nan"), device=dev)
     audio = torch.empty(2, 1920 * frames, device=dev)
-    s4, s5 = torch.empty(128, 960 * frames, device=dev), torch.empty(128, 1920 * frames, device=dev)
-    hip.vae_decode(dw, to_dev(latent, dev), frames, audio, ws, nbytes, stage_outputs=[None] * 3 + [s4, s5])
-    stage = dw.stage[4]
-    x, y, h = (torch.empty(128, 1920 * frames, device=dev) for _ in range(3))
-    hip.snake_conv_transpose1d(s4, 128, 960 * frames, stage.upsample.weight, 128, 2,
+    ci, c, stride = binding.VAE_IN_WIDTH[s], binding.VAE_OUT_WIDTH[s], binding.VAE_STRIDES[s]
+    t_in = frames * int(np.prod(binding.VAE_STRIDES[:s]))
+    t = t_in * stride
+    outputs = [None] * 5
+    outputs[s - 1], outputs[s] = torch.empty(ci, t_in, device=dev), torch.empty(c, t, device=dev)
+    hip.vae_decode(dw, to_dev(latent, dev), frames, audio, ws, nbytes, stage_outputs=outputs)
+    stage = dw.stage[s]
+    x, y, h = (torch.empty(c, t, device=dev) for _ in range(3))
+    hip.snake_conv_transpose1d(outputs[s - 1], ci, t_in, stage.upsample.weight, c, stride,
                                alpha_log=stage.activation.alpha_log, beta_log=stage.activation.beta_log,
-                               bias=stage.upsample.bias, padding=1, y=x)
+                               bias=stage.upsample.bias, padding=(stride + 1) // 2, y=x)
     for unit, dil in zip(stage.residual, (1, 3, 9)):
-        hip.vae_residual_unit(x, 128, 1920 * frames, unit, dil, y, h)
+        hip.vae_residual_unit(x, c, t, unit, dil, y, h)
         x, y = y, x
     torch.cuda.synchronize()
-    return from_dev(s5), from_dev(x)
+    return from_dev(outputs[s]), from_dev(x)
 
 
 @pytest.mark.parametrize("what", ["x nan", "h inf", "h large", "x large", "w0 inf", "w0 nan", "w0 3.4e38", "w1 inf", "w1 nan"])
@@ -297,7 +407,7 @@ def test_unit_special_values(hip, binding, dev, oracle, what):
     else:
         unit["conv" + where[1]][0][17, 5, 0] = np.float32(value)
     dw, keep = device_weights(hip, binding, dev, w)
-    got, plain = _last_stage(hip, binding, dev, w, dw, latent, frames)
+    got, plain = _stage(hip, binding, dev, w, dw, latent, frames, 4)
     nan = np.isnan(plain)
     assert np.array_equal(np.isnan(got), nan)
     inf = np.isinf(plain)
@@ -344,7 +454,7 @@ def test_tiny_operands(hip, dev, oracle, kw, direct, xs, ws):
     """Inputs or weights (or their products) that are all so small that the parts
     would lose bits: as close to the exact sums as the F32 launch, in the 2-norm
     relative to them (10 % and the smallest F32 steps allowed)."""
-    c, c_out, t, stride = (256, 256, 20000, 1) if kw != 2 else (512, 256, 3000, 4)
+    c, c_out, t, stride = (256, 256, 20000, 1) if kw != 2 else (512, 256, 4300, 4)
     if kw == 2:
         x, w, _, _, _ = _t_case(oracle, c, c_out, t, stride, 41)
     else:
