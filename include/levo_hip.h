@@ -113,24 +113,29 @@ int levo_hip_snake_conv1d(const float * x, int64_t x_stride, int64_t c_in, int64
                           int64_t padding, int64_t dilation, const float * residual, int64_t residual_stride,
                           float * y, int64_t y_stride, levo_hip_stream_t stream);
 
-/* Floats of workspace levo_hip_snake_conv1d_split uses at most for an output
- * of c_out x t_out: four partial sums of the output, rows padded to a
- * multiple of 4 floats; < 0 if invalid. */
+/* Floats of workspace for levo_hip_snake_conv1d_split with an output of c_out x
+ * t_out: four partial sums of the output, rows padded to a multiple of 4
+ * floats; < 0 if invalid. A larger one has room for more partial sums of a
+ * small grid and for the split weights of a short, wide convolution. */
 int64_t levo_hip_snake_conv1d_split_workspace_floats(int64_t c_out, int64_t t_out);
 
 /* levo_hip_snake_conv1d (the same arguments, results and errors) with a
  * device workspace of workspace_floats floats (16-byte aligned, overlapping
  * none of the tensors). When the output has fewer 128 x 128 tiles than the
  * GPU has compute units, the input channels are split over up to four
- * workgroups per tile (up to 32 in a grid of fewer than 64 tiles; as many
- * partial sums as the workspace holds), each
- * writing its partial sum to the workspace, and a second launch adds the
- * partials in split order, then the bias and the residual. The result is
- * deterministic; it differs from levo_hip_snake_conv1d's by the F32 rounding
- * of the other summation order. Large launches of more than 128 output
- * channels (kernel 1, 3 or 7, (kernel - 1) * dilation <= 64) run on the bf16
- * matrix cores with every F32 operand as an exact sum of three bf16 values, no
- * further from the exact result than the F32 sums; the workspace then holds
+ * workgroups per tile (up to 32 where the GPU has five compute units and more
+ * for each tile; as many partial sums as the workspace holds), each writing
+ * its partial sum to the workspace, and a second launch adds the partials in
+ * split order, then the bias and the residual. The result is deterministic;
+ * it differs from levo_hip_snake_conv1d's by the F32 rounding of the other
+ * summation order. Large launches of more than 128 output channels (kernel 1,
+ * 3 or 7, (kernel - 1) * dilation <= 64, sums of four terms and more) run on
+ * the bf16 matrix cores where that is estimated to be faster, with every F32
+ * operand as a sum of three bf16 values, exact from 2^-110 up: over the sums
+ * of a convolution no further from the exact result than the F32 launch, whose
+ * infinities and NaN it has. (Tiles of values all below 2^-90, and with values
+ * whose products may overflow, are summed in F32, slowly; among larger values
+ * ones below 2^-110 keep only the bits above 2^-133.) The workspace then holds
  * the split weights (6 bytes each) and the partial sums. Otherwise a grid that
  * already fills the GPU, c_out <= 4 or too small a workspace run
  * levo_hip_snake_conv1d's path unchanged. Same reference call sites as
@@ -162,16 +167,18 @@ int levo_hip_conv_transpose1d_pack_weights(const float * weight, float * packed,
  * SnakeBeta parameters as in levo_hip_snake_conv1d (NULL: none);
  * packed_weight from levo_hip_conv_transpose1d_pack_weights; bias [c_out] or
  * NULL; y: F32 [c_out][y_stride] with (t_in + 1) * stride - 2 * padding
- * samples. The sum is accumulated on the F32 matrix cores in another order
- * than ggml's, so y agrees with the reference to F32 rounding. */
+ * samples. The sum is accumulated in F32 in another order than ggml's, on the
+ * matrix cores or, up to 16 columns q over 512 channels and more, by FMAs, so
+ * y agrees with the reference to F32 rounding. */
 int levo_hip_snake_conv_transpose1d(const float * x, int64_t x_stride, int64_t c_in, int64_t t_in,
                                     const void * alpha_log, const void * beta_log, levo_hip_type param_type,
                                     const float * packed_weight, int64_t c_out, int64_t stride, const float * bias,
                                     int64_t padding, float * y, int64_t y_stride, levo_hip_stream_t stream);
 
-/* Floats of workspace levo_hip_snake_conv_transpose1d_split uses at most:
- * four partial sums of every phase's t_in + 1 output columns, rows padded to
- * a multiple of 4 floats; < 0 if invalid. */
+/* Floats of workspace for levo_hip_snake_conv_transpose1d_split: four partial
+ * sums of every phase's t_in + 1 output columns, rows padded to a multiple of
+ * 4 floats; < 0 if invalid. A larger one has room for more, as for
+ * levo_hip_snake_conv1d_split. */
 int64_t levo_hip_snake_conv_transpose1d_split_workspace_floats(int64_t c_out, int64_t t_in, int64_t stride);
 
 /* levo_hip_snake_conv_transpose1d (the same arguments, results and errors)
@@ -180,8 +187,10 @@ int64_t levo_hip_snake_conv_transpose1d_split_workspace_floats(int64_t c_out, in
  * stride phases) than the GPU has compute units, the input channels are
  * split over up to four (32) workgroups per tile and phase, as
  * levo_hip_snake_conv1d_split does, and a second launch adds each output
- * sample's partial sums in split order, then the bias. Large launches run on
- * the bf16 matrix cores as levo_hip_snake_conv1d_split's do. Deterministic; it
+ * sample's partial sums in split order, then the bias. Large launches of more
+ * than 128 rows (output channels times stride) run on the bf16 matrix cores as
+ * levo_hip_snake_conv1d_split's do; the ones of up to 16 columns that
+ * levo_hip_snake_conv_transpose1d sums by FMAs need no workspace. Deterministic; it
  * differs from levo_hip_snake_conv_transpose1d by the F32 rounding of the
  * other summation order. Same reference call sites. */
 int levo_hip_snake_conv_transpose1d_split(const float * x, int64_t x_stride, int64_t c_in, int64_t t_in,
@@ -251,17 +260,17 @@ int64_t levo_hip_vae_decode_workspace_bytes(int64_t frames);
  * [64][frames] F32 to audio [2][frames * 1920] F32, with the reference's
  * hyper-parameters (latent 64, widths 2048 -> 1024 -> 512 -> 256 -> 128 ->
  * 128, strides 10, 6, 4, 4, 2, dilations 1, 3, 9). 37 fused SnakeBeta +
- * convolution steps (input conv, 7 per stage, output conv):
- * the 128-channel residual units (stages 4 and 5) are one launch each, as
- * levo_hip_vae_residual_unit runs them; a convolution whose grid would
- * leave compute units idle runs split-K (levo_hip_snake_conv1d_split) with
- * one more combine launch, its partial sums in the free tail of a workspace
- * buffer, and large ones run on the bf16 matrix cores (one more launch that
- * splits their weights into free workspace). None of the activations leaves the device, the caller's
- * workspace (16-byte aligned, levo_hip_vae_decode_workspace_bytes) holds
- * them. Every weight the
- * reference's validate_weights requires (src/levo-vae.cpp:56-78) must be
- * non-null. stage_outputs, when non-null, holds 5 device pointers (each may
+ * convolution steps (input conv, 7 per stage, output conv): the 128-channel
+ * residual units (stages 4 and 5) are one launch each, on the F32 matrix cores
+ * as levo_hip_vae_residual_unit runs them up to 6103 samples, on the bf16 ones
+ * (levo_hip_snake_conv1d_split) from there; a convolution whose grid would
+ * leave compute units idle runs split-K with one more combine launch, its
+ * partial sums in the free tail of a workspace buffer, and large ones run on
+ * the bf16 matrix cores. Each bf16 launch has one more before it, which splits
+ * its weights into free workspace. None of the activations leaves the device,
+ * the caller's workspace (16-byte aligned, levo_hip_vae_decode_workspace_bytes)
+ * holds them. Every weight the reference's validate_weights requires
+ * (src/levo-vae.cpp:56-78) must be non-null. stage_outputs, when non-null, holds 5 device pointers (each may
  * be null): stage s's output [width_s][frames * prod(strides[0..s])] is
  * copied there, the reference's capture_stages tensors. Every convolution
  * agrees with the reference to F32 rounding; so does the composition. The

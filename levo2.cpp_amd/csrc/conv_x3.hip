@@ -1,14 +1,17 @@
-// The decoder's convolutions on the bf16 matrix cores without giving up F32:
-// every F32 operand v is the exact sum of three bf16 values, hi + mid + lo
-// (each the round-to-nearest bf16 of what the ones before leave; 8 + 8 + 8
-// significand bits, F32's exponent range), and a product a * b is
+// The decoder's convolutions on the bf16 matrix cores without giving up F32
+// (the three-way split of Henry, Tang and Heinecke, "Leveraging the bfloat16
+// Artificial Intelligence Datatype For Higher-Precision Computations", 2019):
+// every F32 operand v of 2^-110 and up is the exact sum of three bf16 values,
+// hi + mid + lo (each the round-to-nearest bf16 of what the ones before leave; 8
+// + 8 + 8 significand bits), and a product a * b is
 //   hi hi + (hi mid + mid hi) + mid mid + (hi lo + lo hi)
-// in F32 accumulators of v_mfma_f32_32x32x16_bf16. The three products left out
-// (mid lo, lo mid, lo lo) are below 2^-25 |a b|, less than the F32 rounding of
-// a single product. The five small products have accumulators of their own, so
-// the large sum rounds once per 16 terms (the F32 MFMA: once per 4): against
-// float64 the results lie 1.9 to 2.7 times closer than the F32 launches' (512
-// channels, k = 7: 2.0e-7 against 5.4e-7 in the 2-norm).
+// in F32 accumulators of v_mfma_f32_32x32x16_bf16. Of the products left out, mid
+// lo and lo mid are below 2^-25 |a b| each and below 2^-24 together, about the F32
+// rounding of a single product. The five small products have accumulators of
+// their own, so the large sum rounds once per 16 terms (the F32 MFMA: once per
+// 4): against float64 the results lie 1.5 to 3.2 times closer than the F32
+// launches' on sums of four terms and more (512 channels, k = 7: 2.0e-7 against
+// 5.4e-7 in the 2-norm); shorter ones stay with those.
 //
 // What bounds it: the matrix pipe's power. Six bf16 MFMAs take the place of
 // work that costs 16 times their cycles in F32, 417 TFLOP/s of F32 sums at the
@@ -166,12 +169,6 @@ __device__ __forceinline__ uint32_t wave_range(uint32_t r) {
 
 __device__ __forceinline__ float param_at(const void * p, int32_t f16, int i) {
     return f16 ? h2f(static_cast<const uint16_t *>(p)[i]) : static_cast<const float *>(p)[i];
-}
-
-__device__ __forceinline__ float snake_fast(float x, const snake_param & q, bool & slow) {
-    const float m = x * q.alpha;
-    slow |= !(__builtin_fabsf(m) <= kSinSqFastMax);
-    return x + div_by(sin_sq_reduced(m), q.beta, q.rbeta);
 }
 
 // Parameters of a wave-uniform channel by scalar loads: the pack launch wrote
@@ -479,7 +476,7 @@ __device__ __forceinline__ void unit_tail(const x3_kernel_params & p, u32x4 * ld
                         const unit_row & ri = info[32 * wave + acc_row(u + q, hl)];
                         float h = acc[2 * half + j][u + q];
                         if (c.bias) h = h + ri.bias0;
-                        v[q] = exact ? snake(h, ri.post) : snake_fast(h, ri.post, slow);
+                        v[q] = exact ? snake(h, ri.post) : snake_reduced(h, ri.post, slow);
                     }
 #pragma unroll
                     for (int q = 0; q < 4; ++q) largest = __builtin_fmaxf(largest, __builtin_fabsf(v[q]));
@@ -670,7 +667,7 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
             v[q] = inside && ci + q < c.c_in ? xr[m][q] : 0.0f;
             if (SNAKE) {
                 const snake_param sp = scalar_param(p.pre, ci + q);
-                v[q] = exact ? snake(v[q], sp) : snake_fast(v[q], sp, slow);
+                v[q] = exact ? snake(v[q], sp) : snake_reduced(v[q], sp, slow);
             }
         }
         largest = __builtin_fmaxf(__builtin_fmaxf(largest, __builtin_fabsf(v[0])), __builtin_fabsf(v[1]));
@@ -938,7 +935,7 @@ __global__ __launch_bounds__((x3_shape<KW, FUSE>::THREADS), 2) void x3_conv_kern
                         float sv[16];
                         bool slow = false;
 #pragma unroll
-                        for (int u = 0; u < 16; ++u) sv[u] = snake_fast(v[u], info[32 * wave + acc_row(u, hl)].post, slow);
+                        for (int u = 0; u < 16; ++u) sv[u] = snake_reduced(v[u], info[32 * wave + acc_row(u, hl)].post, slow);
                         if (slow) {
 #pragma unroll
                             for (int u = 0; u < 16; ++u) sv[u] = snake(v[u], info[32 * wave + acc_row(u, hl)].post);

@@ -527,22 +527,18 @@ __global__ __launch_bounds__(kThreads) void snake_conv1d_kernel(const conv_param
     conv_epilogue<true>(p.splits > 1 ? split_target(p, tl.z) : p, lds, acc, tid, h, vh, g, m, t0, co0, phase);
 }
 
-__device__ __forceinline__ float snake_reduced(float x, const snake_param & q, bool & slow) {
-    const float m = x * q.alpha;
-    slow |= !(__builtin_fabsf(m) <= kSinSqFastMax);
-    return x + div_by(sin_sq_reduced(m), q.beta, q.rbeta);
-}
-
 // ---- narrow output (c_out <= 4): the decoder's 128 -> 2 output conv -------
 //
 // A 128-row matrix-core tile would compute 2 useful rows, so narrow outputs
 // take a VALU kernel instead: a workgroup owns 256 J output samples (thread
-// tid the samples tid + 256 j, j < J) and walks the input channels in chunks
-// (of 8, or with J = 1, where the time is one workgroup's walk, of 32). A chunk's raw input rows (halo included) and weights are
-// loaded into registers while the previous chunk is summed, then SnakeBeta is
-// applied once per element on the way into LDS; the weights sit in LDS
-// (zero past c_out) and are read at wave-uniform addresses. Every output
-// channel is summed with FMAs over (ci, k) in ascending order.
+// tid the samples tid + 256 j, j < J) and walks the input channels in chunks of
+// 8; with J = 1, where the time is one workgroup's walk, four groups of 256
+// threads each take every fourth chunk. A chunk's raw input rows (halo included)
+// and weights are loaded into registers while the previous chunk is summed, then
+// SnakeBeta is applied once per element on the way into LDS; the weights sit in
+// LDS (zero past c_out) and are read at wave-uniform addresses. Every output
+// channel is summed with FMAs over (ci, k) in ascending order, by each group over
+// its chunks, the groups' sums in group order.
 constexpr int kNarrowMaxSpan = 512;  // (kernel - 1) * dilation
 template <int J>
 constexpr int narrow_row_loads() {  // per row and thread
@@ -563,7 +559,7 @@ struct narrow_regs {
 };
 
 template <int KW, int NCO, int J>
-__device__ __forceinline__ void narrow_load(const conv_params & p, int ci0, int64_t tb, bool inside, int tid,
+__device__ __forceinline__ void narrow_load(const conv_params & p, int ci0, int64_t tb, int tid,
                                             narrow_regs<KW, NCO, J> & r) {
     // clamped and unconditional, masked where they are staged: a branch around
     // each load would have each waited for by itself
@@ -601,7 +597,7 @@ __global__ __launch_bounds__(kThreads * narrow_groups<J>()) void snake_conv_narr
     const int64_t tb = t0 - p.pad;
     const bool inside = tb >= 0 && tb + width <= p.t_in;
     narrow_regs<KW, NCO, J> r;
-    narrow_load<KW, NCO, J>(p, kNarrowCI * grp, tb, inside, tid, r);
+    narrow_load<KW, NCO, J>(p, kNarrowCI * grp, tb, tid, r);
     if (p.snake) {
         for (int c = threadIdx.x; c < p.c_in; c += kThreads * G) {
             const float al = p.param_f16 ? h2f(static_cast<const uint16_t *>(p.alpha_log)[c])
@@ -648,7 +644,7 @@ __global__ __launch_bounds__(kThreads * narrow_groups<J>()) void snake_conv_narr
         for (int i = 0; i < narrow_regs<KW, NCO, J>::NW; ++i)
             if (tid + kThreads * i < NCO * kNarrowCI * KW) ws[tid + kThreads * i] = r.w[i];
         __syncthreads();
-        if (base + kNarrowCI * G < p.c_in) narrow_load<KW, NCO, J>(p, ci0 + kNarrowCI * G, tb, inside, tid, r);  // in flight
+        if (base + kNarrowCI * G < p.c_in) narrow_load<KW, NCO, J>(p, ci0 + kNarrowCI * G, tb, tid, r);  // in flight
         const int nc = min(kNarrowCI, p.c_in - ci0);
         for (int c = 0; c < nc; ++c) {
             const float * row = xs + c * width + tid;
@@ -1421,10 +1417,10 @@ int64_t conv_lds_bytes(int64_t c_in, int64_t table_ch, int64_t dil, bool snake, 
 
 // Splits of a launch of `wgs` workgroups (tiles times stride phases) over
 // `chunks` K chunks of CI channels. A grid with fewer workgroups than CUs
-// splits up to kMaxSplits ways (two workgroups per CU), a grid of fewer than 64
-// up to kMaxThinSplits ways (one per CU), where its time is one workgroup's walk
-// through K: 1024 channels x 70 samples, k = 7, 8 tiles: 172 us in 4 splits, 45 us
-// in the 22 that a decode of 7 frames has space for. A larger grid splits
+// splits up to kMaxSplits ways (two workgroups per CU), one that has five CUs and
+// more for each workgroup up to kMaxThinSplits ways (one per CU), where its time
+// is one workgroup's walk through K: 1024 channels x 70 samples, k = 7, 8 tiles:
+// 172 us in 4 splits, 45 us in the 22 that a decode of 7 frames has space for. A larger grid splits
 // in two when that evens its last round: with w workgroups per CU (two when
 // the launch's LDS fits twice in a CU, one otherwise; a split halves the
 // SnakeBeta table) the launch takes ceil(wgs / (w CUs)) rounds of whole
@@ -1536,10 +1532,8 @@ int try_x3(const conv_params & p, int kw, int64_t splits, float * ws, int64_t ws
     return launch_x3(c, kw, ws, ws + floats, ws_floats - floats, st, what);
 }
 
-// levo_hip_snake_conv1d, and with a workspace the split-K form when the grid
-// would leave compute units idle: up to two workgroups per CU (at most
-// kMaxSplits splits), each split at least two K chunks, as many partial
-// slices as the workspace holds.
+// levo_hip_snake_conv1d, and with a workspace the bf16 form (try_x3) or the
+// split-K one (choose_splits) where they take it.
 int conv1d_entry(const float * x, int64_t x_stride, int64_t c_in, int64_t t_in, const void * alpha_log,
                  const void * beta_log, levo_hip_type param_type, const float * weight, int64_t c_out,
                  int64_t kernel, const float * bias, int64_t padding, int64_t dilation, const float * residual,

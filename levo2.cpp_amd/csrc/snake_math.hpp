@@ -85,6 +85,14 @@ __device__ __forceinline__ float snake(float x, const snake_param & q) {
     return x + d;                   // ggml_add(input, .)
 }
 
+// The same by the reduced form alone; `slow` is set where its argument is
+// beyond that (the caller then evaluates snake).
+__device__ __forceinline__ float snake_reduced(float x, const snake_param & q, bool & slow) {
+    const float m = x * q.alpha;
+    slow |= !(__builtin_fabsf(m) <= kSinSqFastMax);
+    return x + div_by(sin_sq_reduced(m), q.beta, q.rbeta);
+}
+
 // The per-channel parameters from the log-domain values
 // (src/levo-audio-ops.cpp:146-148: exp, then scale_bias(., 1, 1e-9)).
 __device__ __forceinline__ snake_param make_snake_param(float alpha_log, float beta_log) {

@@ -1,7 +1,7 @@
 """Split-K SnakeBeta + Conv1d (levo_hip_snake_conv1d_split): the input
-channels of each 128 x 128 output tile split over up to four workgroups,
-their partial sums combined in split order by a second launch, then the
-bias and the residual (the epilogue of conv_1d_f32 and run_residual,
+channels of each 128 x 128 output tile split over up to four workgroups in
+the queried workspace, their partial sums combined in split order by a
+second launch, then the bias and the residual (the epilogue of conv_1d_f32 and run_residual,
 src/levo-audio-ops.cpp:56-87, src/levo-vae.cpp:91-100).
 
 Bars (F32 max|a - b| / max(|b|, 1)): <= 1e-5 against the same convolution
@@ -14,8 +14,10 @@ oracle's) 1.1e-5 and the three split partial sums 6.6e-6, so the split
 result differs from the oracle by up to the sum of two F32 errors while
 lying closer to the exact convolution than either; two calls bit-identical
 (the combine adds in a fixed order);
-without a workspace, with a grid that fills the GPU or with fewer K chunks
-than splits need, bit-identical to levo_hip_snake_conv1d. Shapes: the
+without a workspace, with a grid that fills the GPU (of launches too small for
+the bf16 form, test_gpu_conv_x3.py, or short of space for its split weights)
+or with fewer K chunks than splits need, bit-identical to
+levo_hip_snake_conv1d. Shapes: the
 decoder's stage 1 at a 10.08 s window (1024 channels x 2520 samples, k = 7
 at dilation 9 and k = 1 with the residual: 160 tiles), the input conv
 (64 -> 2048 channels, 2 K chunks per split), a partial last chunk, ragged
