@@ -1509,10 +1509,15 @@ double f32_launch_us(const conv_params & p, int kw, int64_t splits) {
 
 // The bf16-split form of p (kernel kw, p.o_stride phases) where it takes the
 // convolution: its packed weights at the front of `pack` (or of the
-// workspace), its partial sums in the rest of it. Returns kNotX3
-// with nothing launched where it does not. Of 1690 shapes timed in either form, 12
-// take the slower one by more than 2 % (the worst by 15 %, 253 for 219 us).
+// workspace), its partial sums in the rest of it. Returns kNotX3 with nothing
+// launched where it does not. F32 has to be estimated 1.5 % faster, as the bf16
+// form is the closer one to the exact result: of 1690 shapes timed in either form,
+// 10 take the slower one by more than 2 % (the worst by 15 %, 253 for 219 us) and 19
+// of stage 1's upsampler at 135 to 252 frames the closer one by 7 % (290 for 270 us;
+// in a decode, where F32 finds its weights cold, 296 for 285, and the audio's error
+// against float64 is 6.7e-7 rather than 7.3e-7).
 constexpr int kNotX3 = 1;
+constexpr double kF32Gain = 1.015;
 
 int try_x3(const conv_params & p, int kw, int64_t splits, float * ws, int64_t ws_floats,
            const scratch_span & pack, hipStream_t st, const char * what) {
@@ -1523,10 +1528,10 @@ int try_x3(const conv_params & p, int kw, int64_t splits, float * ws, int64_t ws
     const double f32_us = f32_launch_us(p, kw, splits);
     if (pack.p != nullptr && pack.floats >= floats) {
         const int64_t part = pack.floats - floats;
-        if (x3_us(c, kw, part) >= f32_us) return kNotX3;
+        if (x3_us(c, kw, part) >= kF32Gain * f32_us) return kNotX3;
         return launch_x3(c, kw, pack.p, pack.p + floats, part, st, what);
     }
-    if (ws == nullptr || ws_floats < floats || x3_us(c, kw, ws_floats - floats) >= f32_us) return kNotX3;
+    if (ws == nullptr || ws_floats < floats || x3_us(c, kw, ws_floats - floats) >= kF32Gain * f32_us) return kNotX3;
     // the F32 launch may leave alone what a workspace shares with a tensor
     if (meets_tensor(p, kw, ws, ws_floats)) return kNotX3;
     return launch_x3(c, kw, ws, ws + floats, ws_floats - floats, st, what);
