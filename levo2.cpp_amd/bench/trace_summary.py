@@ -37,6 +37,12 @@ counters: waves, instructions per wave by kind, wave lifetime and the share
 of it spent issuing VALU work:
 
     python3 levo2.cpp_amd/bench/trace_summary.py --issue <sq_counter_collection.csv> <probe stdout> > issue.md
+
+With --vae-issue, the same per kernel and grid of the last decode in a run of
+`bench.py --only vae` with SQ_INSTS_MFMA in SQ_INSTS_SALU's place, and the
+share of the launch that the matrix cores are busy:
+
+    python3 levo2.cpp_amd/bench/trace_summary.py --vae-issue <sq_counter_collection.csv> > issue.md
 """
 from __future__ import annotations
 
@@ -293,6 +299,32 @@ def issue(sq_csv: str, probe_log: str) -> list[str]:
     return rows
 
 
+MFMA_CYCLES = 32  # v_mfma_f32_32x32x16_bf16 on its SIMD
+
+
+def vae_issue(sq_csv: str) -> list[str]:
+    """Per kernel and grid of the last decode: instructions per wave, the share
+    of a wave's lifetime spent issuing VALU work, and the bf16 MFMAs' cycles
+    per SIMD over the launch's SQ-busy cycles per shader engine."""
+    per, what = defaultdict(dict), {}
+    for r in csv.DictReader(open(sq_csv)):
+        if "levo_hip::" in r["Kernel_Name"]:
+            did = int(r["Dispatch_Id"])
+            per[did][r["Counter_Name"]] = float(r["Counter_Value"])
+            what[did] = (short_name(r["Kernel_Name"]), int(r["Grid_Size"]) // int(r["Workgroup_Size"]))
+    ends = [d for d in sorted(per) if "narrow" in what[d][0]]  # the output conv ends a decode
+    launches = {what[d]: per[d] for d in sorted(per) if ends[-2] < d <= ends[-1]}
+    rows = ["| kernel | grid (WGs) | VALU / wave | MFMA / wave | VMEM rd / wave | LDS / wave | "
+            "VALU-active share of lifetime | matrix cores busy |", "|---|---:|---:|---:|---:|---:|---:|---:|"]
+    for (name, wgs), c in launches.items():
+        w = c["SQ_WAVES"]
+        mfma = c["SQ_INSTS_MFMA"] * MFMA_CYCLES / N_SIMDS / (c["SQ_BUSY_CYCLES"] / N_SE) if "x3_conv" in name else 0.0
+        rows.append(f"| `{name}` | {wgs} | {c['SQ_INSTS_VALU'] / w:.0f} | {c['SQ_INSTS_MFMA'] / w:.0f} | "
+                    f"{c['SQ_INSTS_VMEM_RD'] / w:.0f} | {c['SQ_INSTS_LDS'] / w:.0f} | "
+                    f"{c['SQ_ACTIVE_INST_VALU'] / c['SQ_WAVE_CYCLES']:.2f} | {f'{mfma:.2f}' if mfma else '—'} |")
+    return rows
+
+
 if __name__ == "__main__":
     if sys.argv[1] == "--issue":
         print("\n".join(issue(sys.argv[2], sys.argv[3])))
@@ -300,6 +332,8 @@ if __name__ == "__main__":
         print("\n".join(traffic(*sys.argv[2:6])))
     elif sys.argv[1] == "--vae-trace":
         print("\n".join(vae_trace(sys.argv[2])))
+    elif sys.argv[1] == "--vae-issue":
+        print("\n".join(vae_issue(sys.argv[2])))
     elif sys.argv[1] == "--vae":
         print("\n".join(vae_traffic(*sys.argv[2:6])))
     else:

@@ -17,7 +17,7 @@
 // work that costs 16 times their cycles in F32, 417 TFLOP/s of F32 sums at the
 // nominal clock; MFMAs alone on random data hold 1.82 PFLOP/s (the clock falls),
 // 303 TFLOP/s of sums. 512 channels x 60000, k = 7: 2.1 ms and 104 TFLOP/s with
-// the F32 MFMA, 0.94 ms and 235 TFLOP/s here. The weights' way from L2 is 22 %
+// the F32 MFMA, 0.95 ms and 231 TFLOP/s here. The weights' way from L2 is 22 %
 // of the time and the staging 16 % (timed with each left out).
 //
 // As an implicit GEMM: rows R (output channels; for a transposed convolution
@@ -42,8 +42,8 @@
 // hi hi sums have accumulators of their own, so where one is not finite it is
 // the output as it stands: an infinite or NaN operand makes it what the F32 sum
 // is, and what the small products did does not matter (a decode of 252 frames, all
-// of it NaN in the end: 10.7 ms with the look through the tiles' inputs, 7.2 ms for
-// an ordinary one; F32 launches 16 and 13.5 ms). What that does not cover
+// of it NaN in the end: 10.6 ms with the look through the tiles' inputs, 7.1 ms for
+// an ordinary one; F32 launches 15.9 and 13.5 ms). What that does not cover
 // is summed again in plain F32, by the workgroup whose tile it is (f32_needed):
 // sums that are not finite where a finite product may overflow (its parts'
 // products overflow apart, or only the first does) or an operand is so small
